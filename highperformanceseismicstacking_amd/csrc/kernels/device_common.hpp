@@ -21,6 +21,9 @@ constexpr int kMaxWindow = 32;  // MAX_WINDOW_SIZE, common/include/gpu/interface
 // into a __shared__ array is a generic pointer, and code that merges it with a global
 // one falls back to flat loads, which go through the vector memory path.
 using LdsFloat = __attribute__((address_space(3))) float;
+// Two floats in LDS read by one 8-byte access.
+using LdsPairValue = __attribute__((ext_vector_type(2))) float;
+using LdsPair = const volatile __attribute__((address_space(3))) LdsPairValue;
 
 // Wave segment (eval.hpp): kSeg samples per wave in LDS.
 constexpr int kSeg = 128;
@@ -39,30 +42,33 @@ enum ErrorCode {  // gpu_error_code, common/include/gpu/interface.h:12-18
 // operations on every float input (for the division: for this dt), and fall back to the
 // library operations otherwise (see fast_index_verified()).
 //
-// sqrt: v_sqrt_f32 is within one ulp; of s and its two neighbours the correctly rounded
-// root is picked from the signs of the exact residuals x - s'*s (one FMA each).
-// sqrt_rn_big: that sequence alone, for inputs known to be 0 or >= 2^-96 (below, the
-// residual products can underflow).
-// sqrt_rn: inputs below 2^-96 (negative ones included) are first scaled by 2^64, exactly,
-// into that range, and the root by 2^-32 back (exact: the root of a positive float is
-// >= 2^-75, a normal number).  The scaling runs only when some active lane of the wave
-// has such an input (a wave-uniform branch); it is the identity for the other lanes.
+// sqrt: y = v_rsq_f32(x), g = x*y and h = y/2 approximate sqrt(x) and 1/(2 sqrt(x)); one
+// step with the exact residual, g + (x - g*g)*h, lands on the correctly rounded root.  Five
+// operations, 16 issue cycles (v_rsq_f32 takes eight of them) against 32 for picking among
+// v_sqrt_f32's neighbours with two compares and selects, which this replaces: the index
+// chain of the staged CMP loop went from 100 to 68 cycles per trace and candidate with it.
+// sqrt_rn_big: that sequence alone, for normal inputs from 2^-96 up.  Outside them it gives
+// a NaN, an infinity or a value below 2^-47 (0 and +inf give a NaN).
+// sqrt_rn: every input.  When some active lane of the wave has one outside [2^-96, inf) (a
+// wave-uniform branch), inputs are scaled by 2^64 where they are small, exactly, and the
+// root by 2^-32 back (exact: the root of a positive float is >= 2^-75, a normal number),
+// and 0, -0 and +inf are their own roots.
 __device__ __forceinline__ float sqrt_rn_big(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float s_dn = __int_as_float(__float_as_int(s) - 1);
-    const float s_up = __int_as_float(__float_as_int(s) + 1);
-    const float r_dn = __builtin_fmaf(-s_dn, s, x);
-    const float r_up = __builtin_fmaf(-s_up, s, x);
-    float r = r_dn <= 0.0f ? s_dn : s;
-    r = r_up > 0.0f ? s_up : r;
-    return r;
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    const float h = 0.5f * y;
+    const float d = __builtin_fmaf(-g, g, x);
+    return __builtin_fmaf(d, h, g);
 }
 
 __device__ __forceinline__ float sqrt_rn(float x) {
+    // normal inputs from 2^-96 up, as unsigned bit patterns (negative ones are larger)
+    const bool in = __float_as_uint(x) - 0x0f800000u < 0x70000000u;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!in) == 0, 1)) return sqrt_rn_big(x);
     const bool small = x < 0x1.0p-96f;
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(small) == 0, 1)) return sqrt_rn_big(x);
-    const float r = sqrt_rn_big(__builtin_amdgcn_ldexpf(x, small ? 64 : 0));
-    return __builtin_amdgcn_ldexpf(r, small ? -32 : 0);
+    float r = sqrt_rn_big(__builtin_amdgcn_ldexpf(x, small ? 64 : 0));
+    r = __builtin_amdgcn_ldexpf(r, small ? -32 : 0);
+    return x == 0.0f || x == INFINITY ? x : r;
 }
 
 // t / dt from inv = RN(1/dt): q = t*inv, then one correction with the exact residual.
@@ -146,9 +152,10 @@ struct TraceGeom {
 //   OCT    oct/linear_search.cu:84-98
 // t0sq is t0*t0 rounded, hoisted out of the trace loop.  FAST: square roots by sqrt_rn.
 // FAST (used only with tau >= 1 and dt >= 2^-40, see fast_index_verified()): the CMP and
-// ZO-CRS square root is the traveltime itself, so a radicand below 2^-96 -- the only
-// inputs where sqrt_rn_big may differ from sqrtf -- gives t < 2^-48 <= dt, t/dt < 1, and
-// no window with tau >= 1 accepts it either way; the small-input branch is not needed.
+// ZO-CRS square root is the traveltime itself, so a radicand below 2^-96 or +inf -- the
+// inputs where sqrt_rn_big differs from sqrtf -- gives t < 2^-47 or +inf with sqrtf and
+// such a t or a NaN with sqrt_rn_big; no window with tau >= 1 accepts either.  SHIFT: a
+// shift is added to t before the window test, so the root has to be right for every input.
 // ZO-CRS in two parts, the reference's expression in its own operation order: the
 // midpoint part (t0 + A*dm)^2 + B*dm*dm, then + C*h^2 and the square root.  The first
 // depends on the trace's midpoint only, so a loop over a CMP's traces can keep it.
@@ -157,28 +164,33 @@ __device__ __forceinline__ float zocrs_mid_part(float t0, float dm, const Candid
     return tmp * tmp + k.p2 * dm * dm;
 }
 
-template <bool FAST>
+template <bool FAST, bool SHIFT>
+__device__ __forceinline__ float sqrt_time(float x) {
+    if constexpr (!FAST) return sqrtf(x);
+    else if constexpr (SHIFT) return sqrt_rn(x);
+    else return sqrt_rn_big(x);
+}
+
+template <bool FAST, bool SHIFT = false>
 __device__ __forceinline__ bool zocrs_time_from(float mid_part, float c_h2, float *t) {
     const float tmp = mid_part + c_h2;
     if (tmp >= 0) {
-        if constexpr (FAST) *t = sqrt_rn_big(tmp);
-        else *t = sqrtf(tmp);
+        *t = sqrt_time<FAST, SHIFT>(tmp);
         return true;
     }
     return false;
 }
 
-template <int MODEL, bool FAST = false>
+template <int MODEL, bool FAST = false, bool SHIFT = false>
 __device__ __forceinline__ bool traveltime(const TraceGeom &tg, float t0, float t0sq, float m0,
                                            float h0, float apm, const Candidate &k, float *t,
                                            bool *reject) {
     *reject = false;
     if constexpr (MODEL == HSS_CMP) {
-        if constexpr (FAST) *t = sqrt_rn_big(t0sq + k.c * tg.h2);
-        else *t = sqrtf(t0sq + k.c * tg.h2);
+        *t = sqrt_time<FAST, SHIFT>(t0sq + k.c * tg.h2);
         return true;
     } else if constexpr (MODEL == HSS_ZOCRS) {
-        return zocrs_time_from<FAST>(zocrs_mid_part(t0, tg.m - m0, k), k.c * tg.h2, t);
+        return zocrs_time_from<FAST, SHIFT>(zocrs_mid_part(t0, tg.m - m0, k), k.c * tg.h2, t);
     } else {
         float mh;
         int err = oct_displaced_midpoint<FAST>(tg.h, h0, t0, m0, k.c, k.p1, &mh);

@@ -262,9 +262,10 @@ __device__ __forceinline__ void evaluate_n(const EvalCtx &e, float t0, float t0s
                     ok = oct_traveltime<FASTIDX>(ot, oc[c], e.m0, e.apm, &t, &r);
                 else if constexpr (MODEL == HSS_ZOCRS) {
                     r = false;
-                    ok = zocrs_time_from<FASTIDX>(zmid[c], k[c].c * tg.h2, &t);
+                    ok = zocrs_time_from<FASTIDX, SHIFT>(zmid[c], k[c].c * tg.h2, &t);
                 } else
-                    ok = traveltime<MODEL, FASTIDX>(tg, t0, t0sq, e.m0, e.h0, e.apm, k[c], &t, &r);
+                    ok = traveltime<MODEL, FASTIDX, SHIFT>(tg, t0, t0sq, e.m0, e.h0, e.apm, k[c],
+                                                           &t, &r);
                 // counted per wave (the callers add the count of active lanes only)
                 rej += (unsigned)__builtin_popcountll(__builtin_amdgcn_ballot_w64(r & on[c] & active));
                 if constexpr (SHIFT) t = t + shift;
@@ -310,7 +311,7 @@ __device__ __forceinline__ void evaluate_n(const EvalCtx &e, float t0, float t0s
                     for (int c = 0; c < CPL; ++c) {
                         const int rel = kk[c] - e.tau - b + par;
                         const bool fits = (unsigned)rel <= (unsigned)(kSeg - 1 - W);
-                        if (serve[c] & fits) acc[c].add_lds(seg + rel, f[c], e.w);
+                        if (serve[c] & fits) acc[c].add_lds(seg + rel, f[c], e.w, c);
                         rest[c] = serve[c] & !fits;
                     }
                 };
@@ -342,7 +343,7 @@ __device__ __forceinline__ void evaluate_n(const EvalCtx &e, float t0, float t0s
                 const float *row = (const float *)e.samples + trace0 - (size_t)e.tau;
 #pragma unroll
                 for (int c = 0; c < CPL; ++c) {
-                    if (use[c]) acc[c].add_row(row, (unsigned)kk[c], f[c], e.w);
+                    if (use[c]) acc[c].add_row(row, (unsigned)kk[c], f[c], e.w, c);
                 }
             } else if constexpr (W > 0) {
                 // 16-bit samples, per-lane reads of whole words (add16) from the trace's
@@ -354,7 +355,7 @@ __device__ __forceinline__ void evaluate_n(const EvalCtx &e, float t0, float t0s
                 for (int c = 0; c < CPL; ++c) {
                     if (use[c])
                         acc[c].template add16<STORAGE, FACTORED16>(roww, rpar, (unsigned)kk[c],
-                                                                   f[c], sc);
+                                                                   f[c], sc, c);
                 }
             } else {
 #pragma unroll

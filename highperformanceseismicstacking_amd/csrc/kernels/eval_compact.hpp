@@ -140,13 +140,13 @@ __device__ __forceinline__ void evaluate_oct_compact(const EvalCtx &e, float t0,
                         const size_t trace0 = ((size_t)rec.off_hi << 32) | (size_t)rec.off_lo;
                         if constexpr (STORAGE == HSS_F32) {
                             const float *row = (const float *)e.samples + trace0 - (size_t)e.tau;
-                            acc[c].add_row(row, (unsigned)kk, f, e.w);
+                            acc[c].add_row(row, (unsigned)kk, f, e.w, c);
                         } else if constexpr (W > 0) {
                             const size_t row = trace0 - (size_t)e.tau;
                             const unsigned rpar = (unsigned)row & 1u;
                             const uint32_t *roww =
                                 (const uint32_t *)((const uint16_t *)e.samples + (row - rpar));
-                            acc[c].template add16<STORAGE>(roww, rpar, (unsigned)kk, f, rec.sc);
+                            acc[c].template add16<STORAGE>(roww, rpar, (unsigned)kk, f, rec.sc, c);
                         } else {
                             acc[c].add(rd, trace0 + (size_t)(kk - e.tau), f, rec.sc, scaled, e.w);
                         }

@@ -1,7 +1,9 @@
 // Exhaustive check of the short correctly-rounded sequences of device_common.hpp.
 //
 // sqrt_rn(x) must equal sqrtf(x) for every non-negative float (and +inf) and be a NaN for
-// every negative one, and
+// every negative one; sqrt_rn_big(x), the traveltime of CMP and ZO-CRS, must equal sqrtf(x)
+// for every x in [2^-96, inf), and outside give nothing that a window with tau >= 1 and
+// dt >= 2^-40 accepts (a NaN, an infinity or a value below 2^-47); and
 // div_rn(t, dt, RN(1/dt)) must equal t/dt for every float t wherever a window with
 // tau >= 1 could accept either value: 1 <= t/dt < 2e9 (a window needs k = (int)(t/dt) >= tau,
 // window_index()).  Below that range the two may differ -- for |t| < ~2^-103 the residual
@@ -31,6 +33,12 @@ __global__ __launch_bounds__(256) void verify_index_ops_kernel(float dt, float i
             // same bits for x >= 0 (and -0); a NaN for x < 0, as sqrtf gives
             const float a = sqrt_rn(x);
             if (x >= 0.0f ? __float_as_uint(a) != __float_as_uint(sqrtf(x)) : a == a) bad++;
+            const float c = sqrt_rn_big(x);
+            if (x >= 0x1.0p-96f && x < INFINITY) {
+                if (__float_as_uint(c) != __float_as_uint(sqrtf(x))) bad++;
+            } else if (fabsf(c) >= 0x1.0p-47f && fabsf(c) < INFINITY) {
+                bad++;
+            }
         }
         const float e = x / dt;
         const float f = div_rn(x, dt, inv);
@@ -57,7 +65,7 @@ std::map<std::pair<int, unsigned>, bool> verify_cache;  // completed checks only
 // the sequences: both answer false (the library operations, the same bits) and cache
 // nothing, so the next call outside capture runs the check.
 bool fast_index_verified(float dt, int tau, hipStream_t stream) {
-    // tau >= 1: no window accepts t/dt < 1; dt >= 2^-40: a traveltime below 2^-48 (a
+    // tau >= 1: no window accepts t/dt < 1; dt >= 2^-40: a traveltime below 2^-47 (a
     // radicand below 2^-96, where sqrt_rn_big may differ from sqrtf) has t/dt < 1
     if (tau < 1 || !(dt >= 0x1.0p-40f)) return false;
     int dev = 0;

@@ -104,6 +104,60 @@ constexpr int kKahanChunk = 16;
 static_assert((kKahanChunk & (kKahanChunk - 1)) == 0 && kKahanChunk <= 64,
               "the chunk must be a power of two dividing 64");
 
+// Two neighbouring window values as HSS_FAST and HSS_KAHAN sum them: d = y1 - y0,
+// u = fma(d, f, y0), A += u, den = fma(u, u, den), each the same operation the plain
+// expressions give, in registers chosen by hand.
+//
+// What bounds the window sums is VALU issue, and on gfx950 that depends on the registers:
+// an FP32 add, subtract, multiply or FMA whose sources are vector registers issues in two
+// cycles per wave, but an FMA whose three sources all lie in even or all in odd registers
+// takes four, as does any operation with a scalar-register source (measured with
+// independent chains at 4 waves per SIMD: 2.5 against 4.9 cycles of a nominal 2.4 GHz; the
+// sources of an FMA modulo 2 are all that matters).  den = fma(u, u, den) is thus fast only
+// when u and den differ in parity, and the compiler, which does not know, gets a third of
+// a window's FMAs wrong.  Here the differences go to even registers, f sits in an odd one
+// (so fma(d, f, y0) is fast wherever y0 is), the values u go to odd ones and den sits in an
+// even one: eight fast operations.  `slot` is 0 or 1 (a constant after inlining): the
+// candidates of a lane that are summed in one loop keep den and f in registers of their own.
+__device__ __forceinline__ void window_pair(float &A0, float &A1, float &den, float y0, float y1,
+                                            float y2, float f, int slot) {
+#define HSS_WINDOW_PAIR(DEN, F)                            \
+    __asm__("v_sub_f32 v2, %4, %3\n\t"                     \
+            "v_sub_f32 v4, %5, %4\n\t"                     \
+            "v_fma_f32 v3, v2, %6, %3\n\t"                 \
+            "v_fma_f32 v5, v4, %6, %4\n\t"                 \
+            "v_add_f32 %0, %0, v3\n\t"                     \
+            "v_fmac_f32 %2, v3, v3\n\t"                    \
+            "v_add_f32 %1, %1, v5\n\t"                     \
+            "v_fmac_f32 %2, v5, v5"                        \
+            : "+v"(A0), "+v"(A1), "+{" DEN "}"(den)        \
+            : "v"(y0), "v"(y1), "v"(y2), "{" F "}"(f)      \
+            : "v2", "v3", "v4", "v5")
+    if (slot == 0)
+        HSS_WINDOW_PAIR("v6", "v7");
+    else
+        HSS_WINDOW_PAIR("v8", "v9");
+#undef HSS_WINDOW_PAIR
+}
+
+// The same for one value (the last of an odd window).
+__device__ __forceinline__ void window_single(float &A0, float &den, float y0, float y1, float f,
+                                              int slot) {
+#define HSS_WINDOW_SINGLE(DEN, F)                     \
+    __asm__("v_sub_f32 v2, %3, %2\n\t"                \
+            "v_fma_f32 v3, v2, %4, %2\n\t"            \
+            "v_add_f32 %0, %0, v3\n\t"                \
+            "v_fmac_f32 %1, v3, v3"                   \
+            : "+v"(A0), "+{" DEN "}"(den)             \
+            : "v"(y0), "v"(y1), "{" F "}"(f)          \
+            : "v2", "v3")
+    if (slot == 0)
+        HSS_WINDOW_SINGLE("v6", "v7");
+    else
+        HSS_WINDOW_SINGLE("v8", "v9");
+#undef HSS_WINDOW_SINGLE
+}
+
 template <int W, int VARIANT>
 struct Window {
     static constexpr int N = W > 0 ? W : kMaxWindow;
@@ -165,6 +219,40 @@ struct Window {
         step_d(j, y0, y1 - y0, f);
     }
 
+    // The window whose samples are y[0..W] (compiled window sizes).
+    template <class Samples>
+    __device__ __forceinline__ void sum(const Samples &y, float f, int slot) {
+        static_assert(W > 0, "a compiled window size");
+        if constexpr (VARIANT == HSS_EXACT) {
+#pragma unroll
+            for (int j = 0; j < W; ++j) step(j, y[j], y[j + 1], f);
+        } else {
+#pragma unroll
+            for (int j = 0; j + 1 < W; j += 2)
+                window_pair(A[j], A[j + 1], den, y[j], y[j + 1], y[j + 2], f, slot);
+            if constexpr (W & 1) window_single(A[W - 1], den, y[W - 1], y[W], f, slot);
+        }
+    }
+
+    // A window in LDS, row[0..W], without counting its trace in `used`.
+    __device__ __forceinline__ void sum_lds(const LdsFloat *row, float f, int w, int slot) {
+        if constexpr (W > 0) {
+            float y[W + 1];
+#pragma unroll
+            for (int j = 0; j <= W; ++j) y[j] = row[j];
+            sum(y, f, slot);
+        } else {
+            float y1 = row[0];
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                if (j >= w) continue;
+                const float y0 = y1;
+                y1 = row[j + 1];
+                step(j, y0, y1, f);
+            }
+        }
+    }
+
     // Adds the w interpolated values starting at sample `base` of the flat sample array.
     template <class Reader>
     __device__ __forceinline__ void add(const Reader &rd, size_t base, float f, float scale,
@@ -185,8 +273,17 @@ struct Window {
     // FP32 samples of one trace: row[k .. k+w] with `row` wave-uniform (the trace's first
     // sample minus tau) and k the lane's sample index, so the loads take a scalar base and
     // a 32-bit lane offset.
-    __device__ __forceinline__ void add_row(const float *row, unsigned k, float f, int w) {
+    __device__ __forceinline__ void add_row(const float *row, unsigned k, float f, int w,
+                                            int slot = 0) {
         const float *p = row + k;
+        if constexpr (W > 0) {
+            float y[W + 1];
+#pragma unroll
+            for (int j = 0; j <= W; ++j) y[j] = p[j];
+            sum(y, f, slot);
+            used++;
+            return;
+        }
         float y1 = p[0];
 #pragma unroll
         for (int j = 0; j < N; ++j) {
@@ -206,7 +303,7 @@ struct Window {
     // kernel holds one form in its trace loop (both would add registers).
     template <int STORAGE, bool FACTORED = true>
     __device__ __forceinline__ void add16(const uint32_t *roww, unsigned rpar, unsigned k,
-                                          float f, float sc) {
+                                          float f, float sc, int slot = 0) {
         static_assert(W > 0, "add16 needs a compiled window size");
         if constexpr (VARIANT != HSS_EXACT && STORAGE == HSS_F16 && FACTORED) {
             // as below, with y1 - y0 formed as fma(y1, one, -y0) = RN(y1 - y0): the same
@@ -234,8 +331,7 @@ struct Window {
         read16<STORAGE, W>(roww, rpar, k, y);
         if constexpr (VARIANT != HSS_EXACT) {
             if constexpr (!FACTORED) {
-#pragma unroll
-                for (int j = 0; j < W; ++j) step(j, y[j], y[j + 1], f);
+                sum(y, f, slot);
                 used++;
                 return;
             }
@@ -260,16 +356,34 @@ struct Window {
         used++;
     }
 
-    // Same as add() for a window already decoded (and scaled) into LDS: row[0..w].
-    __device__ __forceinline__ void add_lds(const LdsFloat *row, float f, int w) {
-        float y1 = row[0];
+    // A window in LDS stored as pairs, at[i] = {sample i, sample i + 1}, without counting its
+    // trace in `used`: samples j and j + 1 are one aligned 8-byte read from at[j].  (8-byte
+    // reads move 217 bytes per clock and CU where the 4-byte reads of a plain row, whose
+    // windows start anywhere, move 120; measured.  Volatile: the compiler would merge two of
+    // them into one ds_read2_b64, which is back at 122.)
+    __device__ __forceinline__ void sum_pairs(LdsPair *at, float f, int w, int slot) {
+        if constexpr (W > 0) {
+            float y[W + 1];
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            if (W == 0 && j >= w) continue;
-            const float y0 = y1;
-            y1 = row[j + 1];
-            step(j, y0, y1, f);
+            for (int j = 0; j < W; j += 2) {
+                const LdsPairValue p = at[j];
+                y[j] = p.x;
+                y[j + 1] = p.y;
+            }
+            sum(y, f, slot);
+        } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                if (j >= w) continue;
+                const LdsPairValue p = at[j];
+                step(j, p.x, p.y, f);
+            }
         }
+    }
+
+    // Same as add() for a window already decoded (and scaled) into LDS: row[0..w].
+    __device__ __forceinline__ void add_lds(const LdsFloat *row, float f, int w, int slot = 0) {
+        sum_lds(row, f, w, slot);
         used++;
     }
 
