@@ -16,10 +16,10 @@ int launch_grid_cmp_staged(const GridArgs &a, int n_slots, int variant, int stor
                               SS = decltype(S)::value;
                 if (cpl == 2 && WW > 0)
                     hipLaunchKernelGGL((grid_staged_kernel<WW, VV, SS, 2>), dim3(blocks),
-                                       dim3(kGridThreads), 0, stream, a);
+                                       dim3(kStagedThreads), 0, stream, a);
                 else
                     hipLaunchKernelGGL((grid_staged_kernel<WW, VV, SS, 1>), dim3(blocks),
-                                       dim3(kGridThreads), 0, stream, a);
+                                       dim3(kStagedThreads), 0, stream, a);
             });
         });
     });

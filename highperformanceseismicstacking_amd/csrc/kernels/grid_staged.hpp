@@ -3,71 +3,90 @@
 // The grid kernel (grid_impl.hpp) lets every wave read its own windows: FP32 lanes with
 // 16-byte loads (the texture-address unit is then the busiest unit after the VALU), 16-bit
 // storage through a per-wave LDS segment that each wave loads and decodes for itself.
-// Here the four waves of a workgroup (one 64-sample t0 tile of a midpoint) take their
+// Here the eight waves of a workgroup (one 64-sample t0 tile of a midpoint) take their
 // candidates in rounds -- round r: wave v evaluates the CPL candidates starting at
-// (4r + v)*CPL, the same candidates in the same order as the grid kernel's wave v -- and
-// walk the midpoint's traces together, a block at a time.  For each trace of a block the
-// workgroup first loads, decodes and scales into LDS the samples that any window of the
-// round can read, then every lane reads its windows from there.  (Blocks of 32 traces;
-// HSS_KAHAN: 16.)
+// (8r + v)*CPL -- and walk the midpoint's traces together, a block at a time.  For each trace
+// of a block the workgroup first loads, decodes and scales into LDS the samples that any
+// window of the round can read, then every lane reads its windows from there.  (Blocks of
+// 32 traces; HSS_KAHAN: 16.)  Eight waves rather than four halve the staging per candidate
+// and the length of a workgroup, and with it the launch's tail: 10.2 -> 9.7 ms on a
+// 150-midpoint line (w = 11, 512 candidates), 52.0 -> 50.9 ms on a 256-midpoint one (FP16,
+// w = 15, 1024 candidates).
 //
 // The staged span of a trace follows from monotonicity (CMP: t = sqrt(t0^2 + c h^2) and
 // every operation of the index chain are nondecreasing in t0 and in c): the smallest
 // window start of the round is at the tile's first t0 and the round's smallest c, the
-// largest at its last t0 and largest c.  A block with a trace whose span exceeds the stage
-// takes direct reads instead.  Each lane adds its traces in the same order with the same
-// operations on the same values as the grid kernel, so the results are the same bits
-// (HSS_KAHAN's chunk boundaries are the same 16-trace blocks).
+// largest at its last t0 and largest c.  When both corners' windows lie inside the trace,
+// every lane's do, and the trace loop is straight-line code: no bounds tests, no lane masks,
+// both candidates' index chains interleaved (lanes past the last sample repeat it).  Traces
+// whose span crosses the trace's ends keep the tests; a trace whose span exceeds the stage
+// is read directly.  Each lane adds its traces in the same order with the same operations
+// on the same values as the grid kernel, so the results are the same bits (HSS_KAHAN's
+// chunk boundaries are the same 16-trace blocks).
+//
+// What bounds it: VALU issue.  On the 256-midpoint line the straight-line loop is 147 VALU
+// instructions per trace and two candidates (120 of them the windows), 322 issue cycles at
+// the rates of window.hpp; the launch takes 395 cycles per trace and two candidates, with
+// the VALU issuing 93% of the time.  Before (four waves, masked lanes, dword stage loads)
+// 485 cycles; 61.0 -> 50.9 ms.
 #pragma once
 
 #include "grid_impl.hpp"
 
 namespace hss {
 
-// Samples staged per trace: 128, loaded by the first two waves (one sample per thread).
-// The C5 line's spans (a 64-sample t0 tile plus the window and the moveout across the
-// round's candidates) fit; a 256-sample stage was 4.7% slower (more LDS per workgroup, one
-// workgroup fewer per CU).
+// Samples staged per trace: 128, four per lane, two traces per wave and load.  The C5 line's spans (a 64-sample t0 tile plus the window and the moveout
+// across the round's candidates) fit; a 256-sample stage was 4.7% slower (more LDS per
+// workgroup, one workgroup fewer per CU).
+constexpr int kStagedWaves = 8;
+constexpr int kStagedThreads = kStagedWaves * kWave;
 constexpr int kStageCap = 128;
-static_assert(kStageCap % kWave == 0 && kStageCap <= kGridThreads, "whole waves load the stage");
+constexpr int kStageLaneSamples = 4;
+constexpr int kStageRowLanes = kStageCap / kStageLaneSamples;  // lanes that load one trace
+constexpr int kStageRowsPerWave = kWave / kStageRowLanes;
 // Traces per stage: 32 (16 KB of LDS; 48 was no faster, 16 was 3% slower on the C5 line),
 // and for HSS_KAHAN its compensation chunk, since its sums are flushed at those fixed
 // trace blocks.
 template <int VARIANT>
 constexpr int stage_traces() { return VARIANT == HSS_KAHAN ? kKahanChunk : 32; }
 
-// Register budget: five waves per SIMD (96 VGPRs), 4% faster than the four the compiler
-// picks by itself on the C5 line and faster than six; HSS_KAHAN keeps the grid kernel's
-// budget.  At 96 registers nothing may be spilled: a spill slot is per-lane memory that
-// stays in L2 beside the traces (5 resident midpoints per XCD at five waves), and the C5
-// launch then read 63 GB and wrote 46 GB instead of about 3 GB.  Hence the running best in
-// LDS, the uniform values in scalar registers and thread_index_here().
-template <int VARIANT, int CPL>
+// Register budget, as waves per SIMD.  A workgroup is two waves per SIMD, so budgets between
+// four and six waves buy nothing.  Windows of up to 11 samples fit six (11 samples spill 28
+// bytes outside the trace loop; 9.57 ms at six against 9.73 at four on a 150-midpoint line),
+// wider ones take four without spills (50.9 against 52.4 ms at six on a 256-midpoint line).
+// Inside the trace loop nothing may be spilled: a spill slot is per-lane memory that stays
+// in L2 beside the traces.  Hence the running best in LDS, the uniform values in scalar
+// registers and thread_index_here().  HSS_KAHAN keeps the grid kernel's budget.
+template <int W, int VARIANT, int CPL>
 constexpr int staged_min_waves() {
-    return VARIANT == HSS_KAHAN ? grid_min_waves<VARIANT, CPL>() : 5;
-}
-
-// The sample index (int)(t/dt) of the index chain, clamped into [-1, 2^24] first (the
-// span only needs the order; lanes use indices inside (lo, hi) of index_bounds()).
-template <bool FAST>
-__device__ __forceinline__ int span_index(float t, float dt, float inv) {
-    float ti;
-    if constexpr (FAST) ti = div_rn(t, dt, inv);
-    else ti = t / dt;
-    ti = fminf(fmaxf(ti, -1.0f), 16777216.0f);  // a NaN becomes -1
-    return (int)ti;
+    if (VARIANT == HSS_KAHAN) return grid_min_waves<VARIANT, CPL>();
+    return W == 0 ? 2 : (W <= 11 ? 6 : 4);
 }
 
 // The running best of each thread, in LDS.
 struct RunBest {
-    float best[kGridThreads];
-    float stack[kGridThreads];
-    int idx[kGridThreads];
+    float best[kStagedThreads];
+    float stack[kStagedThreads];
+    int idx[kStagedThreads];
 };
 
+// What the trace loop needs of one staged trace: h^2 and the LDS address at which sample
+// index k's window starts, minus 8*k.
+struct StagedTrace {
+    float h2;
+    uint32_t row;
+};
+
+// A wave-uniform value in a vector register: an operation with a scalar-register source
+// issues at half the rate of one on vector registers (window.hpp).
+__device__ __forceinline__ float vector_f(float x) {
+    __asm__("" : "+v"(x));
+    return x;
+}
+
 template <int W, int VARIANT, int STORAGE, int CPL>
-__global__ __launch_bounds__(kGridThreads)
-__attribute__((amdgpu_waves_per_eu(staged_min_waves<VARIANT, CPL>(), 8))) void grid_staged_kernel(
+__global__ __launch_bounds__(kStagedThreads)
+__attribute__((amdgpu_waves_per_eu(staged_min_waves<W, VARIANT, CPL>(), 8))) void grid_staged_kernel(
     GridArgs a) {
     using Reader = SampleReader<STORAGE>;
     constexpr bool FASTIDX = W != 0;
@@ -84,22 +103,27 @@ __attribute__((amdgpu_waves_per_eu(staged_min_waves<VARIANT, CPL>(), 8))) void g
     const int s = tile * kWave + lane;
     const int ns = a.e.ns;
     const bool active = s < ns;
-    const float t0 = (float)s * a.e.dt;
+    // lanes past the last sample follow it: they read what it reads and write nothing
+    const float t0 = (float)min(s, ns - 1) * a.e.dt;
     const float t0sq = t0 * t0;
     const EvalCtx e = midpoint_ctx(a.e, a.mbeg, a.mcnt, a.mm0, g);
     const bool scaled = (STORAGE != HSS_F32) && e.scale != nullptr;
     Reader rd{(decltype(Reader::p))e.samples};
     // the tile's first and last t0 (the span's corners)
-    const float t0a = uniform_f((float)(tile * kWave) * e.dt);
-    const float t0b = uniform_f((float)min(tile * kWave + kWave - 1, ns - 1) * e.dt);
+    const float t0a = (float)(tile * kWave) * e.dt;
+    const float t0b = (float)min(tile * kWave + kWave - 1, ns - 1) * e.dt;
     const float t0a_sq = uniform_f(t0a * t0a), t0b_sq = uniform_f(t0b * t0b);
     // the midpoint's [ns][P] slabs of the optional cubes (the host keeps ns * P below 2^32)
     float *const sembl_g = a.sembl ? a.sembl + (size_t)g * ns * a.P : nullptr;
     float *const stack_g = a.stack ? a.stack + (size_t)g * ns * a.P : nullptr;
 
-    constexpr int kStageTraces = stage_traces<VARIANT>();
-    static_assert(kStageTraces <= kWave, "a block's traces are one wave's lanes");
-    __shared__ float stage[kStageTraces][kStageCap];
+    constexpr int ST = stage_traces<VARIANT>();
+    static_assert(2 * ST <= kWave, "a block's span corners are one wave's lanes");
+    static_assert(ST % (kStagedWaves * kStageRowsPerWave) == 0, "whole loads");
+    // stage[jj][i] = samples i and i + 1 of trace jj's span: a window that starts at any i is
+    // (W + 1)/2 aligned 8-byte reads, 16 bytes apart
+    __shared__ alignas(16) float2 stage[ST][kStageCap];
+    __shared__ StagedTrace meta[ST + 1];
     // the lane's running best (first strict maximum over its candidates in order), kept in
     // LDS rather than in registers, which the window sums of two candidates use up; each
     // thread reads and writes only its own slots
@@ -107,52 +131,74 @@ __attribute__((amdgpu_waves_per_eu(staged_min_waves<VARIANT, CPL>(), 8))) void g
     run.best[threadIdx.x] = -1.0f;
     run.stack[threadIdx.x] = 0.0f;
     run.idx[threadIdx.x] = -1;
+    if (threadIdx.x == 0) meta[ST] = StagedTrace{0.0f, 0u};
+    const float dt_v = vector_f(e.dt), inv_v = vector_f(e.inv_dt);
 
-    const int per_round = kGridWaves * CPL;
+    const int per_round = kStagedWaves * CPL;
     const int rounds = (a.P + per_round - 1) / per_round;
     for (int r = 0; r < rounds; ++r) {
-        const int q0 = (r * kGridWaves + wave) * CPL;
-        Candidate k[CPL];
+        const int q0 = (r * kStagedWaves + wave) * CPL;
+        float kc[CPL];
         bool on[CPL];
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             on[c] = q0 + c < a.P;
-            k[c] = load_candidate<HSS_CMP>(a.params, on[c] ? q0 + c : min(q0, a.P - 1));
+            kc[c] = vector_f(a.params[on[c] ? q0 + c : min(q0, a.P - 1)]);
         }
         // the round's range of c (all waves: the same candidates, the same values)
         float cmin = INFINITY, cmax = -INFINITY;
+        bool c_ok = true;  // no NaN among them
         const int qa = r * per_round, qb = min(a.P, qa + per_round);
         for (int q = qa; q < qb; ++q) {
             const float c = a.params[q];
             cmin = fminf(cmin, c);
             cmax = fmaxf(cmax, c);
+            c_ok = c_ok && c == c;
         }
         Window<W, VARIANT> acc[CPL];
 #pragma unroll
         for (int c = 0; c < CPL; ++c) acc[c].reset();
 
-        for (int j0 = 0; j0 < e.cnt; j0 += kStageTraces) {
-            const int nj = min(kStageTraces, e.cnt - j0);
-            // lane jj < nj: trace j0 + jj's geometry, scale and staged span
+        for (int j0 = 0; j0 < e.cnt; j0 += ST) {
+            const int nj = min(ST, e.cnt - j0);
+            // lanes jj and ST + jj < 2*ST: trace j0 + jj's geometry, scale and staged span;
+            // the first of the two works out the span's lower corner, the second its upper
             const int ln = thread_index_here() & (kWave - 1);
-            const bool have = ln < nj;
-            const int ti_l = have ? (e.midx ? e.midx[e.beg + j0 + ln] : e.beg + j0 + ln) : 0;
+            const int tr = ln & (ST - 1);
+            const bool upper = (ln & ST) != 0;
+            const bool have = tr < nj;
+            const int ti_l = have ? (e.midx ? e.midx[e.beg + j0 + tr] : e.beg + j0 + tr) : 0;
             const float h2_l = have ? e.hoff2[ti_l] : 0.0f;
             const float sc_l = (scaled && have) ? e.scale[ti_l] : 1.0f;
-            int base_l = 0, fit_l = 0;
+            int base_l;
+            unsigned long long fit, clean;  // bit jj: trace j0 + jj
             {
-                TraceGeom tg{0.0f, 0.0f, 0.0f};
-                tg.h2 = h2_l;
-                Candidate lo{cmin, 0.0f, 0.0f}, hi{cmax, 0.0f, 0.0f};
-                float ta, tb;
-                bool r0;
-                traveltime<HSS_CMP, FASTIDX>(tg, t0a, t0a_sq, e.m0, e.h0, e.apm, lo, &ta, &r0);
-                traveltime<HSS_CMP, FASTIDX>(tg, t0b, t0b_sq, e.m0, e.h0, e.apm, hi, &tb, &r0);
-                const int ka = span_index<FASTIDX>(ta, e.dt, e.inv_dt);
-                const int kb = span_index<FASTIDX>(tb, e.dt, e.inv_dt);
-                base_l = max(ka - e.tau, 0);
-                // windows run from k - tau to k + tau + 1
-                fit_l = (have && kb + e.tau + 2 - base_l <= kStageCap) ? 1 : 0;
+                const float x = (upper ? t0b_sq : t0a_sq) + (upper ? cmax : cmin) * h2_l;
+                const float t = sqrt_time<FASTIDX, false>(x);
+                float ti;
+                if constexpr (FASTIDX) ti = div_rn(t, e.dt, e.inv_dt);
+                else ti = t / e.dt;
+                // the corner's sample index (the span needs the order only: lanes use
+                // indices inside (lo, hi) of index_bounds()); a corner that has none, or
+                // whose root sqrt_rn_big does not give, stands for the whole trace
+                const bool usable = x >= 0x1.0p-96f && x < INFINITY;
+                const int none = upper ? 1 << 24 : -1;
+                const int k = usable ? (int)fminf(fmaxf(ti, -1.0f), 16777216.0f) : none;
+                const bool in = usable && ti > e.ib.lo && ti < e.ib.hi;
+                const int kx = __shfl_xor(2 * k + (in ? 1 : 0), ST, kWave);
+                const int ka = upper ? (kx >> 1) : k, kb = upper ? k : (kx >> 1);
+                // windows run from k - tau to k + tau + 1, inside the trace
+                const int first = max(ka - e.tau, 0), end = min(kb + e.tau + 2, ns);
+                base_l = min(first, ns - kStageCap);
+                if (STORAGE != HSS_F32 && ((((ti_l & ns) ^ base_l) & 1) != 0))
+                    // 16-bit samples are loaded in aligned words: an even flat index
+                    base_l += base_l < first ? 1 : -1;
+                // (monotone in c only for h^2 >= 0)
+                const bool ok = have && ns >= kStageCap && h2_l >= 0.0f && end - base_l <= kStageCap;
+                fit = __builtin_amdgcn_ballot_w64(ok) & ((1ull << ST) - 1);
+                // every window of the trace lies inside it: no bounds tests
+                clean = W == 0 || !c_ok ? 0
+                                        : __builtin_amdgcn_ballot_w64(in && (kx & 1)) & fit;
             }
             if constexpr (VARIANT == HSS_KAHAN) {
                 if (j0 > 0) {
@@ -160,102 +206,147 @@ __attribute__((amdgpu_waves_per_eu(staged_min_waves<VARIANT, CPL>(), 8))) void g
                     for (int c = 0; c < CPL; ++c) acc[c].flush(e.w);
                 }
             }
-            // The block is staged when every one of its traces fits; otherwise it takes the
-            // direct reads (one read path per loop, chosen for the whole workgroup: every
-            // wave computes the same spans).
-            const unsigned long long want =
-                nj >= kWave ? ~0ull : ((1ull << nj) - 1ull);
-            const bool staged = (__builtin_amdgcn_ballot_w64(fit_l != 0) & want) == want;
-            if (staged && STORAGE == HSS_F32) {
-                // FP32: the samples go from global memory straight into LDS
-                // (global_load_lds_dword: lane l of wave v < kStageCap/64 writes
-                // stage[jj][64 v + l]), no registers in between; a lane past the trace's end
-                // loads nothing (its slot is never read)
-                __syncthreads();  // every wave has read the previous staged block
-                for (int jj = 0; jj < nj; ++jj) {
-                    const int base = __builtin_amdgcn_readlane(base_l, jj);
-                    const int ti = __builtin_amdgcn_readlane(ti_l, jj);
-                    const int i = base + (int)threadIdx.x;
-                    if (i < ns && wave < kStageCap / kWave)
-                        __builtin_amdgcn_global_load_lds(
-                            (const float *)e.samples + (size_t)ti * (size_t)ns + (size_t)i,
-                            (__attribute__((address_space(3))) void *)&stage[jj][wave * kWave], 4,
-                            0, 0);
-                }
-                __syncthreads();  // (the compiler waits for the loads before the barrier)
-            } else if (staged) {
-                // 16-bit: all of the block's loads first, then the decoded and scaled values
-                // into LDS (one wait, not one per trace)
-                float vals[kStageTraces];
+            if (fit != 0) {
+                constexpr int LOADS = ST / (kStagedWaves * kStageRowsPerWave);
+                const size_t off_l = (size_t)ti_l * (size_t)ns + (size_t)(ptrdiff_t)base_l;
+                const int col = (ln & (kStageRowLanes - 1)) * kStageLaneSamples;
+                // The sample after the lane's own four (the last lane's would lie past the
+                // stage, where no window reads)
+                const int after = min(col + kStageLaneSamples, kStageCap - 1);
+                auto row_of = [&](int i) {  // the trace this lane helps load in load i
+                    return (i * kStagedWaves + wave) * kStageRowsPerWave + ln / kStageRowLanes;
+                };
+                auto offset_of = [&](int row) {
+                    return (size_t)(uint32_t)__shfl((int)(off_l >> 32), row, kWave) << 32 |
+                           (uint32_t)__shfl((int)off_l, row, kWave);
+                };
+                // all of the block's loads first, then the (decoded and scaled) samples into
+                // LDS: one wait, not one per trace
+                constexpr bool F32S = STORAGE == HSS_F32;
+                constexpr int RAW = F32S ? kStageLaneSamples + 1 : kStageLaneSamples / 2 + 1;
+                uint32_t raw[LOADS][RAW];
 #pragma unroll
-                for (int jj = 0; jj < kStageTraces; ++jj) {
-                    vals[jj] = 0.0f;
-                    if (jj >= nj) continue;
-                    const int base = __builtin_amdgcn_readlane(base_l, jj);
-                    const int ti = __builtin_amdgcn_readlane(ti_l, jj);
-                    const int i = base + (int)threadIdx.x;  // within the trace: no window reads past ns
-                    if (i < ns && (int)threadIdx.x < kStageCap) vals[jj] = rd((size_t)ti * (size_t)ns + (size_t)i);
+                for (int i = 0; i < LOADS; ++i) {
+                    const int row = row_of(i);
+                    const size_t off = offset_of(row);
+#pragma unroll
+                    for (int q = 0; q < RAW; ++q) raw[i][q] = 0;
+                    if ((fit >> row) & 1) {
+                        if constexpr (F32S) {
+                            const uint32_t *src = (const uint32_t *)e.samples + off;
+#pragma unroll
+                            for (int q = 0; q < RAW - 1; ++q) raw[i][q] = src[col + q];
+                            raw[i][RAW - 1] = src[after];
+                        } else {
+                            const uint32_t *src =
+                                (const uint32_t *)((const uint16_t *)e.samples + off);
+#pragma unroll
+                            for (int q = 0; q < RAW - 1; ++q) raw[i][q] = src[col / 2 + q];
+                            raw[i][RAW - 1] = src[after / 2];
+                        }
+                    }
                 }
                 __syncthreads();  // every wave has read the previous staged block
+                if (wave == 0 && ln < nj)
+                    meta[ln] = StagedTrace{
+                        h2_l, (uint32_t)(size_t)((const LdsFloat *)&stage[0][0]) +
+                                  8u * (uint32_t)(kStageCap * ln - base_l - e.tau)};
 #pragma unroll
-                for (int jj = 0; jj < kStageTraces; ++jj) {
-                    if (jj >= nj) continue;
-                    float v = vals[jj];
-                    // as the wave segments do (a sample past the trace stays 0 and is never read)
-                    if (STORAGE != HSS_F32 || scaled) v = v * bcast(sc_l, jj);
-                    if ((int)threadIdx.x < kStageCap) stage[jj][threadIdx.x] = v;
+                for (int i = 0; i < LOADS; ++i) {
+                    const int row = row_of(i);
+                    float v[kStageLaneSamples + 1];
+                    if constexpr (F32S) {
+#pragma unroll
+                        for (int q = 0; q < RAW; ++q) v[q] = __uint_as_float(raw[i][q]);
+                    } else {
+                        // as the wave segments decode and scale
+                        const float sc = __shfl(sc_l, row, kWave);
+#pragma unroll
+                        for (int q = 0; q <= kStageLaneSamples; ++q) {
+                            const uint32_t d = raw[i][q / 2];
+                            if constexpr (STORAGE == HSS_F16)
+                                v[q] = (float)__builtin_bit_cast(
+                                           _Float16, (uint16_t)((q & 1) ? d >> 16 : d & 0xffffu)) * sc;
+                            else
+                                v[q] = __uint_as_float((q & 1) ? d & 0xffff0000u : d << 16) * sc;
+                        }
+                    }
+                    float4 *dst = (float4 *)&stage[row][col];
+                    dst[0] = float4{v[0], v[1], v[1], v[2]};
+                    dst[1] = float4{v[2], v[3], v[3], v[4]};
                 }
                 __syncthreads();
             }
-            // the lane's sample index, weight and inclusion for trace jj of the block
-            auto index = [&](int jj, int (&kk)[CPL], float (&f)[CPL], bool (&use)[CPL]) {
-                TraceGeom tg{0.0f, 0.0f, 0.0f};
-                tg.h2 = bcast(h2_l, jj);
+            // One read path per loop, chosen for the whole workgroup (every wave computes the
+            // same spans): runs of consecutive traces that are staged with all their windows
+            // inside the trace, staged, or read directly.
+            for (int jj = 0; jj < nj;) {
+                const bool cl = (clean >> jj) & 1, ft = (fit >> jj) & 1;
+                const unsigned long long same = cl ? clean : (ft ? fit & ~clean : ~fit);
+                const int je = min(nj, jj + (int)__builtin_ctzll(~(same >> jj) | (1ull << ST)));
+                if (W > 0 && cl) {
+                    // every lane's windows of both candidates, no masks: index, read, sum
 #pragma unroll
-                for (int c = 0; c < CPL; ++c) {
-                    float t = 0.0f;
-                    bool rj;
-                    const bool ok = traveltime<HSS_CMP, FASTIDX>(tg, t0, t0sq, e.m0, e.h0, e.apm,
-                                                                 k[c], &t, &rj);
-                    const bool in = window_k<FASTIDX>(t, e.dt, e.inv_dt, e.ib, &kk[c], &f[c]);
-                    use[c] = ok & in & active & on[c];
-                }
-            };
-            if (staged) {
-                for (int jj = 0; jj < nj; ++jj) {
-                    // the staged row shifted so that sample index k reads its window start
-                    // k - tau (a workgroup-uniform base: one address operation per window)
-                    const int shift = __builtin_amdgcn_readlane(base_l, jj) + e.tau;
-                    const uint32_t row = (uint32_t)__builtin_amdgcn_readfirstlane(
-                        (int)((uint32_t)(size_t)((const LdsFloat *)&stage[jj][0]) -
-                              4u * (uint32_t)shift));
-                    int kk[CPL];
-                    float f[CPL];
-                    bool use[CPL];
-                    index(jj, kk, f, use);
+                    for (int c = 0; c < CPL; ++c) acc[c].used += (unsigned)(je - jj);
+                    for (; jj < je; ++jj) {
+                        const StagedTrace m = meta[jj];
+                        LdsPair *at[CPL];
+                        float f[CPL];
 #pragma unroll
-                    for (int c = 0; c < CPL; ++c) {
-                        if (use[c])
-                            acc[c].add_lds((const LdsFloat *)(size_t)(row + 4u * (uint32_t)kk[c]),
-                                           f[c], e.w);
+                        for (int c = 0; c < CPL; ++c) {
+                            const float t = sqrt_rn_big(t0sq + kc[c] * m.h2);
+                            const float ti = div_rn(t, dt_v, inv_v);
+                            f[c] = __builtin_amdgcn_fractf(ti);
+                            at[c] = (LdsPair *)(size_t)(m.row + 8u * (uint32_t)(int)ti);
+                        }
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c) {
+                            acc[c].sum_pairs(at[c], f[c], e.w, c);
+                        }
                     }
+                    continue;
                 }
-            } else {
-                for (int jj = 0; jj < nj; ++jj) {
-                    const size_t trace0 = (size_t)__builtin_amdgcn_readlane(ti_l, jj) * (size_t)ns;
-                    const float sc = bcast(sc_l, jj);
-                    int kk[CPL];
-                    float f[CPL];
-                    bool use[CPL];
-                    index(jj, kk, f, use);
+                // the lane's sample index, weight and inclusion
+                auto index = [&](float h2, int (&kk)[CPL], float (&f)[CPL], bool (&use)[CPL]) {
 #pragma unroll
                     for (int c = 0; c < CPL; ++c) {
-                        if (!use[c]) continue;
-                        if constexpr (STORAGE == HSS_F32)
-                            acc[c].add_row((const float *)e.samples + trace0 - (size_t)e.tau,
-                                           (unsigned)kk[c], f[c], e.w);
-                        else
-                            acc[c].add(rd, trace0 + (size_t)(kk[c] - e.tau), f[c], sc, true, e.w);
+                        const float t = sqrt_time<FASTIDX, false>(t0sq + kc[c] * h2);
+                        const bool in =
+                            window_k<FASTIDX>(t, e.dt, e.inv_dt, e.ib, &kk[c], &f[c]);
+                        use[c] = in & active & on[c];
+                    }
+                };
+                int kk[CPL];
+                float f[CPL];
+                bool use[CPL];
+                if (ft) {
+                    for (; jj < je; ++jj) {
+                        const StagedTrace m = meta[jj];
+                        index(m.h2, kk, f, use);
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c) {
+                            if (!use[c]) continue;
+                            acc[c].sum_pairs((LdsPair *)(size_t)(m.row + 8u * (uint32_t)kk[c]),
+                                             f[c], e.w, c);
+                            acc[c].used++;
+                        }
+                    }
+                } else {
+                    for (; jj < je; ++jj) {
+                        const size_t trace0 =
+                            (size_t)__builtin_amdgcn_readlane(ti_l, jj) * (size_t)ns;
+                        const float sc = bcast(sc_l, jj);
+                        index(bcast(h2_l, jj), kk, f, use);
+#pragma unroll
+                        for (int c = 0; c < CPL; ++c) {
+                            if (!use[c]) continue;
+                            if constexpr (STORAGE == HSS_F32)
+                                acc[c].add_row((const float *)e.samples + trace0 - (size_t)e.tau,
+                                               (unsigned)kk[c], f[c], e.w, c);
+                            else
+                                acc[c].add(rd, trace0 + (size_t)(kk[c] - e.tau), f[c], sc, true,
+                                           e.w);
+                        }
                     }
                 }
             }
@@ -289,7 +380,7 @@ __attribute__((amdgpu_waves_per_eu(staged_min_waves<VARIANT, CPL>(), 8))) void g
     float B = -1.0f, BS = 0.0f;
     int BI = -1;
 #pragma unroll
-    for (int v = 0; v < kGridWaves; ++v) {
+    for (int v = 0; v < kStagedWaves; ++v) {
         const int iv = run.idx[v * kWave + ln];
         const float sv = run.best[v * kWave + ln];
         if (iv >= 0 && (sv > B || (sv == B && iv < BI))) {
