@@ -22,67 +22,110 @@
 
 namespace hss {
 
-// 16-bit samples read per lane without LDS (compiled window sizes only, all odd): the
-// (W+1)/2 + 1 aligned 32-bit words around samples e0 .. e0+W, widened to float (not
-// scaled).  FP16: the words shifted by one sample when e0 is odd (v_alignbit), then
-// converted.  BF16: one v_perm_b32 per sample moves its two bytes into the high half of a
-// zero word (selector byte 0x0c gives 0x00), from either word of the pair, so the shift
-// and the widening are one instruction; sample 2i (2i+1) of the window is bytes {1,0}
-// ({3,2}) of the pair for even e0 and bytes {3,2} ({5,4}) for odd e0.  Words q[0 .. NW-2] cover samples
-// a .. a+W (a = e0 rounded down to even), all inside the window or the sample just before
-// it; the last word is needed only for odd e0, where it holds sample e0+W (and the sample
-// after it, inside the same aligned word); for even e0 it re-reads q[NW-2].  The window's
-// first sample e0 is sample rpar + k of the wave-uniform word row `roww` (the row's first
-// sample rounded down to an even sample, i.e. a 4-byte word of the aligned sample array;
-// rpar = 1 when it was odd), so the loads take a scalar base and a 32-bit lane offset.
+// base + a 32-bit byte offset: with a wave-uniform base the load takes the base in scalar
+// registers and the offset as it is, no 64-bit address arithmetic per lane.
+__device__ __forceinline__ const char *at_bytes(const void *base, uint32_t offset) {
+    return (const char *)base + offset;
+}
+
+// All ones for p = 1, 0 for p = 0.
+__device__ __forceinline__ uint32_t p_mask(unsigned p) { return 0u - p; }
+
+// 16-bit samples read per lane without LDS (compiled window sizes only, all odd).  The
+// window's first sample e0 is sample rpar + k of the wave-uniform word row `roww` (the row's
+// first sample rounded down to an even sample, i.e. a 4-byte word of the aligned sample
+// array; rpar = 1 when it was odd), so the loads take a scalar base and a 32-bit lane
+// offset.  Words16 holds the words of samples e0 .. e0+W: for even e0 the (W+1)/2 words from
+// word e0/2 on, for odd e0 one more.  What a kernel that reads windows per lane waits for is
+// the vector cache, which takes every lane's line of every load by itself (an OCT
+// differential evolution ran at 1.1 lines per clock and CU with four loads per window), so
+// the words come in as few loads as possible, none of them past the last word needed: `a`
+// from the window's first word on, and `b`, which starts at the last word of `a` for even e0
+// (p = 0) and right behind it for odd e0 (p = 1).
+template <int W>
+struct Words16 {
+    static_assert(W & 1, "covers an even number of samples");
+    static constexpr int NW = (W + 1) / 2 + 1;
+    static constexpr int NA = NW <= 4 ? 2 : (NW - 1) / 4 * 4;
+    static constexpr int NB = NW - NA;
+    uint32_t a[NA], b[NB];
+    unsigned p;
+
+    __device__ __forceinline__ void load(const uint32_t *roww, unsigned rpar, unsigned k) {
+        const unsigned e0 = rpar + k;
+        p = e0 & 1u;
+        const uint32_t at = (e0 >> 1) << 2;
+        const uint32_t *qa = (const uint32_t *)at_bytes(roww, at);
+        const uint32_t *qb = (const uint32_t *)at_bytes(roww, at + 4u * p) + (NA - 1);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) a[i] = qa[i];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) b[i] = qb[i];
+    }
+
+    // Word i of the window shifted down to start at sample e0 (samples e0 + 2i, e0 + 2i + 1).
+    // v_alignbit shifts by one sample or none; past `a` the operands move by one word with
+    // p, which one v_perm_b32 does in the same step.
+    __device__ __forceinline__ uint32_t shifted(int i, uint32_t sel) const {
+        if (i < NA - 1) return __builtin_amdgcn_alignbit(a[i + 1], a[i], 16u * p);
+        if (i == NA - 1) return __builtin_amdgcn_alignbit(b[0], a[i], 16u * p);
+        return __builtin_amdgcn_perm(b[i - NA + 1], b[i - NA], sel);
+    }
+    // shifted()'s selector: the second word whole (p = 0), or the halves around the boundary
+    __device__ __forceinline__ uint32_t selector() const { return p ? 0x05040302u : 0x07060504u; }
+};
+
+// The window's samples widened to float (not scaled).  BF16: one v_perm_b32 per sample moves
+// its two bytes into the high half of a zero word (selector byte 0x0c gives 0x00), from
+// either word of the pair, so the shift and the widening are one instruction.
 template <int STORAGE, int W>
 __device__ __forceinline__ void read16(const uint32_t *roww, unsigned rpar, unsigned k,
                                        float (&y)[W + 1]) {
-    static_assert(W & 1, "read16 covers an even number of samples");
-    constexpr int NW = (W + 1) / 2 + 1;
-    const unsigned e0 = rpar + k;
-    const unsigned p = e0 & 1u;
-    const uint32_t *q = roww + (e0 >> 1);
-    uint32_t D[NW];
-#pragma unroll
-    for (int i = 0; i < NW - 1; ++i) D[i] = q[i];
-    D[NW - 1] = q[NW - 2 + p];
+    Words16<W> d;
+    d.load(roww, rpar, k);
+    constexpr int NA = Words16<W>::NA;
     if constexpr (STORAGE == HSS_F16) {
+        const uint32_t sel = d.selector();
 #pragma unroll
-        for (int i = 0; i < NW - 1; ++i) {
-            const uint32_t e = __builtin_amdgcn_alignbit(D[i + 1], D[i], 16u * p);
+        for (int i = 0; i < (W + 1) / 2; ++i) {
+            const uint32_t e = d.shifted(i, sel);
             y[2 * i] = (float)__builtin_bit_cast(_Float16, (uint16_t)(e & 0xffffu));
             y[2 * i + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(e >> 16));
         }
     } else {
-        const uint32_t sel_even = 0x01000c0cu | (p ? 0x02020000u : 0u);
-        const uint32_t sel_odd = sel_even + 0x02020000u;
+        // samples 2i and 2i + 1: bytes {1,0} and {3,2} of words i+1:i for even e0, {3,2} and
+        // {5,4} for odd e0; past `a`, where the pair b[i-NA+1]:b[i-NA] is one word lower for
+        // even e0, {5,4} and {7,6}
+        const uint32_t odd = p_mask(d.p) & 0x02020000u;
+        const uint32_t ae = 0x01000c0cu + odd, ao = 0x03020c0cu + odd;
+        const uint32_t be = 0x05040c0cu - odd, bo = 0x07060c0cu - odd;
 #pragma unroll
-        for (int i = 0; i < NW - 1; ++i) {
-            y[2 * i] = __uint_as_float(__builtin_amdgcn_perm(D[i + 1], D[i], sel_even));
-            y[2 * i + 1] = __uint_as_float(__builtin_amdgcn_perm(D[i + 1], D[i], sel_odd));
+        for (int i = 0; i < (W + 1) / 2; ++i) {
+            if (i < NA) {
+                const uint32_t hi = i + 1 < NA ? d.a[i + 1] : d.b[0];
+                y[2 * i] = __uint_as_float(__builtin_amdgcn_perm(hi, d.a[i], ae));
+                y[2 * i + 1] = __uint_as_float(__builtin_amdgcn_perm(hi, d.a[i], ao));
+            } else {
+                const uint32_t hi = d.b[i - NA + 1], lo = d.b[i - NA];
+                y[2 * i] = __uint_as_float(__builtin_amdgcn_perm(hi, lo, be));
+                y[2 * i + 1] = __uint_as_float(__builtin_amdgcn_perm(hi, lo, bo));
+            }
         }
     }
 }
 
-// FP16 samples e0 .. e0+W of one window as halves (the words of read16 shifted by one
-// sample for odd e0, not converted): arithmetic on (float)h[j] then reads each half
-// straight from its word (v_fma_mix_f32) instead of converting it first.
+// FP16 samples e0 .. e0+W of one window as halves (shifted by one sample for odd e0, not
+// converted): arithmetic on (float)h[j] then reads each half straight from its word
+// (v_fma_mix_f32) instead of converting it first.
 template <int W>
 __device__ __forceinline__ void read16_halves(const uint32_t *roww, unsigned rpar, unsigned k,
                                               _Float16 (&h)[W + 1]) {
-    static_assert(W & 1, "read16 covers an even number of samples");
-    constexpr int NW = (W + 1) / 2 + 1;
-    const unsigned e0 = rpar + k;
-    const unsigned p = e0 & 1u;
-    const uint32_t *q = roww + (e0 >> 1);
-    uint32_t D[NW];
+    Words16<W> d;
+    d.load(roww, rpar, k);
+    const uint32_t sel = d.selector();
 #pragma unroll
-    for (int i = 0; i < NW - 1; ++i) D[i] = q[i];
-    D[NW - 1] = q[NW - 2 + p];
-#pragma unroll
-    for (int i = 0; i < NW - 1; ++i) {
-        const uint32_t e = __builtin_amdgcn_alignbit(D[i + 1], D[i], 16u * p);
+    for (int i = 0; i < (W + 1) / 2; ++i) {
+        const uint32_t e = d.shifted(i, sel);
         h[2 * i] = __builtin_bit_cast(_Float16, (uint16_t)(e & 0xffffu));
         h[2 * i + 1] = __builtin_bit_cast(_Float16, (uint16_t)(e >> 16));
     }
@@ -156,6 +199,24 @@ __device__ __forceinline__ void window_single(float &A0, float &den, float y0, f
     else
         HSS_WINDOW_SINGLE("v8", "v9");
 #undef HSS_WINDOW_SINGLE
+}
+
+// Two neighbouring values u0, u1 of a window whose trace scale is factored out:
+// A += sc*u, dn = fma(u, u, dn), in registers of the right parities (window_pair).
+__device__ __forceinline__ void window_pair_scaled(float &A0, float &A1, float &dn, float u0,
+                                                   float u1, float sc, int slot) {
+#define HSS_WINDOW_PAIR_SCALED(DN, SC)                                    \
+    __asm__("v_fmac_f32 %0, %5, %3\n\t"                                   \
+            "v_fmac_f32 %2, %3, %3\n\t"                                   \
+            "v_fmac_f32 %1, %5, %4\n\t"                                   \
+            "v_fmac_f32 %2, %4, %4"                                       \
+            : "+v"(A0), "+v"(A1), "+{" DN "}"(dn)                         \
+            : "{v3}"(u0), "{v5}"(u1), "{" SC "}"(sc))
+    if (slot == 0)
+        HSS_WINDOW_PAIR_SCALED("v6", "v10");
+    else
+        HSS_WINDOW_PAIR_SCALED("v8", "v12");
+#undef HSS_WINDOW_PAIR_SCALED
 }
 
 template <int W, int VARIANT>
@@ -295,6 +356,22 @@ struct Window {
         used++;
     }
 
+    // A window's values value(0) .. value(W-1) without their trace's scale: A_j += sc*u_j and
+    // dn = sum_j u_j^2.
+    template <class Value>
+    __device__ __forceinline__ void sum_scaled(const Value &value, float &dn, float sc, int slot) {
+#pragma unroll
+        for (int j = 0; j + 1 < W; j += 2) {
+            const float u0 = value(j), u1 = value(j + 1);
+            window_pair_scaled(A[j], A[j + 1], dn, u0, u1, sc, slot);
+        }
+        if constexpr (W & 1) {
+            const float u = value(W - 1);
+            A[W - 1] = __builtin_fmaf(sc, u, A[W - 1]);
+            dn = __builtin_fmaf(u, u, dn);
+        }
+    }
+
     // 16-bit samples of one window read per lane (read16), then summed.  FACTORED: the
     // non-exact variants factor the trace's scale `sc` out of the window (a line without
     // scales passes sc = 1).  !FACTORED, for a line stored without scales (BF16: FP32's
@@ -316,13 +393,11 @@ struct Window {
             float one = 1.0f;
             __asm__("" : "+s"(one));
             float dn = 0.0f;
-#pragma unroll
-            for (int j = 0; j < W; ++j) {
+            auto value = [&](int j) {
                 const float d = __builtin_fmaf((float)h[j + 1], one, -(float)h[j]);
-                const float u = __builtin_fmaf(d, f, (float)h[j]);
-                A[j] = __builtin_fmaf(sc, u, A[j]);
-                dn = __builtin_fmaf(u, u, dn);
-            }
+                return __builtin_fmaf(d, f, (float)h[j]);
+            };
+            sum_scaled(value, dn, sc, slot);
             den = __builtin_fmaf(sc * sc, dn, den);
             used++;
             return;
@@ -338,12 +413,8 @@ struct Window {
             // the trace's scale factored out of the window: u = sc * (y0 + frac*(y1 - y0))
             // on the stored values, A_j += sc*u and den += sc^2 * sum_j u^2
             float dn = 0.0f;
-#pragma unroll
-            for (int j = 0; j < W; ++j) {
-                const float u = __builtin_fmaf(y[j + 1] - y[j], f, y[j]);
-                A[j] = __builtin_fmaf(sc, u, A[j]);
-                dn = __builtin_fmaf(u, u, dn);
-            }
+            sum_scaled([&](int j) { return __builtin_fmaf(y[j + 1] - y[j], f, y[j]); }, dn, sc,
+                       slot);
             den = __builtin_fmaf(sc * sc, dn, den);
         } else {
             if constexpr (FACTORED) {
