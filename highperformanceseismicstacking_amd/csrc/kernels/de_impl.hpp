@@ -19,6 +19,7 @@
 #pragma once
 
 #include "eval_compact.hpp"
+#include "eval_runs.hpp"
 #include "grid_impl.hpp"
 #include "launch_util.hpp"
 
@@ -182,7 +183,16 @@ __attribute__((amdgpu_waves_per_eu(de_min_occupancy<MODEL, W, VARIANT>(), 8))) v
     };
 
     __shared__ float seg_lds[kDeWaves][kSegFloats];
-    __shared__ OctTraceRec trace_recs[kDeWaves][kWave];
+    // OCT: the midpoint's offset runs, or (lists without them) the waves' records of a chunk
+    // of traces (uniform over the workgroup)
+    union OctLists {
+        OctRuns runs;
+        OctTraceRec chunk[kDeWaves][kWave];
+    };
+    __shared__ std::conditional_t<de_compact<MODEL, VARIANT>(), OctLists, int> oct_lists;
+    bool by_runs = false;
+    if constexpr (de_compact<MODEL, VARIANT>())
+        by_runs = load_oct_runs(e, STORAGE == HSS_F32 ? 4 : 2, oct_lists.runs);
     constexpr int CPL = de_cpl<MODEL, W, VARIANT>();
     // the individuals a lane evaluates together, from their drawing to their selection
     __shared__ float held[CPL * D][kDeWaves * kWave];
@@ -190,10 +200,14 @@ __attribute__((amdgpu_waves_per_eu(de_min_occupancy<MODEL, W, VARIANT>(), 8))) v
     auto eval = [&](const Candidate (&kc)[CPL], const bool (&on)[CPL], float (&S)[CPL],
                     float (&stk)[CPL]) {
         unsigned rej = 0;  // on the wave's lowest active lane
-        if constexpr (de_compact<MODEL, VARIANT>())
-            evaluate_oct_compact<W, VARIANT, STORAGE, false, CPL>(
-                e, t0, kc, on, 0.0f, active, trace_recs[wave], S, stk, &rej);
-        else if (STORAGE == HSS_BF16 && e.scale == nullptr)
+        if constexpr (de_compact<MODEL, VARIANT>()) {
+            if (by_runs)
+                evaluate_oct_runs<W, VARIANT, STORAGE, false, CPL>(e, oct_lists.runs, t0, kc, on,
+                                                                   0.0f, active, S, stk, &rej);
+            else
+                evaluate_oct_compact<W, VARIANT, STORAGE, false, CPL>(
+                    e, t0, kc, on, 0.0f, active, oct_lists.chunk[wave], S, stk, &rej);
+        } else if (STORAGE == HSS_BF16 && e.scale == nullptr)
             // a BF16 line stored without scales: its windows summed as FP32 windows (one
             // form per code path, chosen outside the trace loop)
             evaluate_n<MODEL, W, VARIANT, STORAGE, false, CPL, kDeSegments, kDeOctKeep, false>(

@@ -155,7 +155,9 @@ struct TraceGeom {
 // ZO-CRS square root is the traveltime itself, so a radicand below 2^-96 or +inf -- the
 // inputs where sqrt_rn_big differs from sqrtf -- gives t < 2^-47 or +inf with sqrtf and
 // such a t or a NaN with sqrt_rn_big; no window with tau >= 1 accepts either.  SHIFT: a
-// shift is added to t before the window test, so the root has to be right for every input.
+// shift n*dt is added to t before the window test, c is 4/v^2 >= 0 and the launcher sees to
+// dt >= 2^-20; a root below 2^-47 then rounds away in the sum (or n is 0 and nothing accepts
+// it), so 0 stands for it.
 // ZO-CRS in two parts, the reference's expression in its own operation order: the
 // midpoint part (t0 + A*dm)^2 + B*dm*dm, then + C*h^2 and the square root.  The first
 // depends on the trace's midpoint only, so a loop over a CMP's traces can keep it.
@@ -167,8 +169,9 @@ __device__ __forceinline__ float zocrs_mid_part(float t0, float dm, const Candid
 template <bool FAST, bool SHIFT>
 __device__ __forceinline__ float sqrt_time(float x) {
     if constexpr (!FAST) return sqrtf(x);
-    else if constexpr (SHIFT) return sqrt_rn(x);
-    else return sqrt_rn_big(x);
+    const float r = sqrt_rn_big(x);
+    if constexpr (SHIFT) return x < 0x1.0p-96f ? 0.0f : r;
+    return r;
 }
 
 template <bool FAST, bool SHIFT = false>

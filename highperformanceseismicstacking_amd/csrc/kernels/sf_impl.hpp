@@ -15,6 +15,7 @@
 
 #include "eval.hpp"
 #include "eval_compact.hpp"
+#include "eval_runs.hpp"
 #include "grid_impl.hpp"
 #include "launch_util.hpp"
 
@@ -52,8 +53,13 @@ constexpr int sf_min_waves() {
     return MODEL == HSS_OCT && VARIANT != HSS_KAHAN && W > 0 && W <= 11 ? 6 : 1;
 }
 
+// Waves per workgroup: OCT eight, so that three workgroups, each with its midpoint's offset
+// runs in LDS, still fill a CU's 24 wave slots of that budget.
+template <int MODEL>
+constexpr int sf_waves() { return MODEL == HSS_OCT ? 8 : kGridWaves; }
+
 template <int MODEL, int W, int VARIANT, int STORAGE>
-__global__ __launch_bounds__(kGridThreads)
+__global__ __launch_bounds__(sf_waves<MODEL>() * kWave)
 __attribute__((amdgpu_waves_per_eu(sf_min_waves<MODEL, W, VARIANT>(), 8))) void sf_semblance_kernel(SfArgs a) {
     constexpr int NP = MODEL == HSS_CMP ? 1 : (MODEL == HSS_ZOCRS ? 3 : 2);
     const int lane = threadIdx.x & (kWave - 1);
@@ -69,8 +75,16 @@ __attribute__((amdgpu_waves_per_eu(sf_min_waves<MODEL, W, VARIANT>(), 8))) void 
     const EvalCtx e = midpoint_ctx(a.e, a.mbeg, a.mcnt, a.mm0, g);
     const float *vp = a.vparams + (size_t)g * NP * ns;
 
-    __shared__ float seg_lds[kGridWaves][kSegFloats];
-    __shared__ OctTraceRec trace_recs[kGridWaves][kWave];
+    constexpr int kWaves = sf_waves<MODEL>();
+    constexpr bool kRuns = MODEL == HSS_OCT && VARIANT != HSS_KAHAN;
+    // OCT: the midpoint's offset runs, or the waves' records of a chunk of traces (eval_runs)
+    union OctLists {
+        OctRuns runs;
+        OctTraceRec chunk[kWaves][kWave];
+    };
+    __shared__ std::conditional_t<kRuns, OctLists, int> oct_lists;
+    bool by_runs = false;
+    if constexpr (kRuns) by_runs = load_oct_runs(e, STORAGE == HSS_F32 ? 4 : 2, oct_lists.runs);
     float best = -1.0f, bstack = 0.0f;
     int bidx = -1;
     unsigned long long rejected = 0;
@@ -78,11 +92,11 @@ __attribute__((amdgpu_waves_per_eu(sf_min_waves<MODEL, W, VARIANT>(), 8))) void 
     // offset when the midpoint's list is grouped by offset (wave-uniform); each lane's
     // candidate comes from its own sample, and the kept terms are per lane all the same
     bool keep = false;
-    if constexpr (MODEL == HSS_OCT) keep = oct_offset_runs_long(e);
+    if constexpr (MODEL == HSS_OCT) keep = by_runs || oct_offset_runs_long(e);
     // a BF16 line stored without scales sums its windows as FP32 windows; both choices are
     // made outside the trace loop, one code path each
     const bool unscaled16 = STORAGE == HSS_BF16 && e.scale == nullptr;
-    for (int q = wave; q < a.nN; q += kGridWaves) {
+    for (int q = wave; q < a.nN; q += kWaves) {
         const int n = (int)a.nvals[q];
         const int sn = s - n;
         const bool valid = active && sn >= 0 && sn < ns;
@@ -102,20 +116,25 @@ __attribute__((amdgpu_waves_per_eu(sf_min_waves<MODEL, W, VARIANT>(), 8))) void 
         auto eval = [&](auto keep_c, auto factored_c) {
             evaluate<MODEL, W, VARIANT, STORAGE, true, kSfSegments, decltype(keep_c)::value,
                      decltype(factored_c)::value>(e, t0n, t0n * t0n, k, (float)n * e.dt, valid,
-                                                  seg_lds[wave], &S, &stk, &rej);
+                                                  nullptr, &S, &stk, &rej);
         };
         using T = std::true_type;
         using F = std::false_type;
         bool walked = false;
         if constexpr (MODEL == HSS_OCT && VARIANT != HSS_KAHAN) {
             if (keep) {
-                // each lane walks only the traces its own aperture keeps (the compacted
-                // walk of differential evolution; the same sums in the same order)
+                // each lane walks only the traces its own aperture keeps (the walks of
+                // differential evolution; the same sums in the same order)
                 const Candidate kc[1] = {k};
                 const bool on[1] = {true};
                 float s1[1], t1[1];
-                evaluate_oct_compact<W, VARIANT, STORAGE, true, 1>(
-                    e, t0n, kc, on, (float)n * e.dt, valid, trace_recs[wave], s1, t1, &rej);
+                if (by_runs)
+                    evaluate_oct_runs<W, VARIANT, STORAGE, true, 1>(
+                        e, oct_lists.runs, t0n, kc, on, (float)n * e.dt, valid, s1, t1, &rej);
+                else
+                    evaluate_oct_compact<W, VARIANT, STORAGE, true, 1>(
+                        e, t0n, kc, on, (float)n * e.dt, valid, oct_lists.chunk[wave], s1, t1,
+                        &rej);
                 S = s1[0];
                 stk = t1[0];
                 walked = true;
@@ -153,7 +172,7 @@ __attribute__((amdgpu_waves_per_eu(sf_min_waves<MODEL, W, VARIANT>(), 8))) void 
     }
     float B, BS;
     int BI;
-    merge_bests<kGridWaves>(best, bstack, bidx, wave, lane, 1, &B, &BS, &BI);
+    merge_bests<kWaves>(best, bstack, bidx, wave, lane, 1, &B, &BS, &BI);
     if (wave != 0 || !active) return;
     float *res = a.result + (size_t)g * 3 * ns;
     res[s] = B;
@@ -168,10 +187,13 @@ int launch_sf(const SfArgs &a, int n_mid, int variant, int storage, hipStream_t 
     if (blocks == 0) return HSS_OK;
     int rc = dispatch_storage(storage, [&](auto S) {
         st = dispatch_variant(variant, [&](auto V) {
-            dispatch_window(a.e.w, fast_index_verified(a.e.dt, a.e.tau, stream), [&](auto Wc) {
+            // (dt: see sqrt_time)
+            const bool fast = a.e.dt >= 0x1.0p-20f && fast_index_verified(a.e.dt, a.e.tau, stream);
+            dispatch_window(a.e.w, fast, [&](auto Wc) {
                 hipLaunchKernelGGL((sf_semblance_kernel<MODEL, decltype(Wc)::value,
                                                         decltype(V)::value, decltype(S)::value>),
-                                   dim3(blocks), dim3(kGridThreads), 0, stream, a);
+                                   dim3(blocks), dim3(sf_waves<MODEL>() * kWave), 0, stream,
+                                   a);
             });
         });
     });
