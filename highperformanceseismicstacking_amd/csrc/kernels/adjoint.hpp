@@ -14,6 +14,7 @@
 #pragma once
 
 #include "eval.hpp"
+#include "eval_runs.hpp"
 #include "launch_util.hpp"
 
 namespace hss {
@@ -215,6 +216,84 @@ __device__ __forceinline__ bool traveltime_grad(const TraceGeom &tg, float t0, f
     }
 }
 
+// The window sums of S and of its gradient for one lane, and their reduction.
+template <int D, int W>
+struct GradSums {
+    static constexpr int N = W > 0 ? W : kMaxWindow;
+    float A[N], G[N][D], H[D];
+    float den;
+    unsigned used;
+
+    __device__ __forceinline__ void reset() {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            A[j] = 0.0f;
+#pragma unroll
+            for (int m = 0; m < D; ++m) G[j][m] = 0.0f;
+        }
+#pragma unroll
+        for (int m = 0; m < D; ++m) H[m] = 0.0f;
+        den = 0.0f;
+        used = 0;
+    }
+
+    // One trace's window y[0..w] at weight f, with gi = (dt/dtheta)/dt.
+    __device__ __forceinline__ void add(const float (&y)[N + 1], float f, const float (&gi)[D],
+                                        int w) {
+        float eu = 0.0f;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            if (W == 0 && j >= w) continue;
+            const float y0 = y[j];
+            const float y1 = y[j + 1];
+            const float d = y1 - y0;
+            const float u = __builtin_fmaf(d, f, y0);
+            A[j] += u;
+            den = __builtin_fmaf(u, u, den);
+            eu = __builtin_fmaf(u, d, eu);
+#pragma unroll
+            for (int m = 0; m < D; ++m) G[j][m] = __builtin_fmaf(d, gi[m], G[j][m]);
+        }
+#pragma unroll
+        for (int m = 0; m < D; ++m) H[m] = __builtin_fmaf(eu, gi[m], H[m]);
+        used++;
+    }
+
+    __device__ __forceinline__ void reduce(int w, float *S, float *stack, float *grad) const {
+        float sem = 0.0f, stk = 0.0f;
+        float gr[D];
+#pragma unroll
+        for (int m = 0; m < D; ++m) gr[m] = 0.0f;
+        if (used > 0 && den > 0.0f) {
+            float num = 0.0f, lin = 0.0f;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                if (W == 0 && j >= w) continue;
+                num = __builtin_fmaf(A[j], A[j], num);
+                lin += A[j];
+            }
+            const float uden = (float)used * den;
+            sem = num / uden;
+            stk = lin / (float)(used * (unsigned)w);
+            const float scl = 2.0f / uden;
+#pragma unroll
+            for (int m = 0; m < D; ++m) {
+                float a = 0.0f;
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    if (W == 0 && j >= w) continue;
+                    a = __builtin_fmaf(A[j], G[j][m], a);
+                }
+                gr[m] = scl * (a - sem * (float)used * H[m]);
+            }
+        }
+        *S = sem;
+        *stack = stk;
+#pragma unroll
+        for (int m = 0; m < D; ++m) grad[m] = gr[m];
+    }
+};
+
 // S, stack and dS/dtheta for one lane's own parameter point.  FMA arithmetic (as
 // HSS_FAST); per-lane windows are read with per-lane loads.  Every lane of the wave must
 // call it (the trace geometry is broadcast across the wave).
@@ -228,17 +307,8 @@ __device__ __forceinline__ void evaluate_grad(const EvalCtx &e, float t0, float 
     using Reader = SampleReader<STORAGE>;
     const bool scaled = (STORAGE != HSS_F32) && e.scale != nullptr;
     const Reader rd{(decltype(Reader::p))e.samples};
-    float A[N], G[N][D], H[D];
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-        A[j] = 0.0f;
-#pragma unroll
-        for (int m = 0; m < D; ++m) G[j][m] = 0.0f;
-    }
-#pragma unroll
-    for (int m = 0; m < D; ++m) H[m] = 0.0f;
-    float den = 0.0f;
-    unsigned used = 0;
+    GradSums<D, W> sums;
+    sums.reset();
     const int lane = threadIdx.x & (kWave - 1);
     // OCT: the point's dual terms of the current half offset, kept while consecutive
     // traces share the offset's bit pattern (a wave-uniform test) when the list comes in
@@ -307,60 +377,83 @@ __device__ __forceinline__ void evaluate_grad(const EvalCtx &e, float t0, float 
                 for (int j = 0; j <= N; ++j)
                     y[j] = (j <= e.w) ? rd(trace0 + (size_t)first + j) * sc : 0.0f;
             }
-            float eu = 0.0f;
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                if (W == 0 && j >= e.w) continue;
-                const float y0 = y[j];
-                const float y1 = y[j + 1];
-                const float d = y1 - y0;
-                const float u = __builtin_fmaf(d, f, y0);
-                A[j] += u;
-                den = __builtin_fmaf(u, u, den);
-                eu = __builtin_fmaf(u, d, eu);
-#pragma unroll
-                for (int m = 0; m < D; ++m) G[j][m] = __builtin_fmaf(d, gi[m], G[j][m]);
-            }
-#pragma unroll
-            for (int m = 0; m < D; ++m) H[m] = __builtin_fmaf(eu, gi[m], H[m]);
-            used++;
+            sums.add(y, f, gi, e.w);
         }
     }
-    float sem = 0.0f, stk = 0.0f;
-    float gr[D];
+    sums.reduce(e.w, S, stack, grad);
+}
+
+// evaluate_grad for an OCT midpoint whose list comes in offset runs (eval_runs.hpp): the
+// forward and the dual terms once per run, then each lane walks the traces its aperture
+// keeps.  The same windows, values and sums in the same order.
+template <int W, int STORAGE>
+__device__ __forceinline__ void evaluate_grad_runs(const EvalCtx &e, const OctRuns &runs, float t0,
+                                                   const Candidate &k, bool active, float *S,
+                                                   float *stack, float *grad) {
+    constexpr int D = 2;
+    constexpr int N = W > 0 ? W : kMaxWindow;
+    constexpr bool FASTIDX = W != 0;
+    GradSums<D, W> sums;
+    sums.reset();
+    const OctCand oc = oct_cand(t0, e.h0, k);
+    Dual<2> c, sl;
+    oct_seed_duals(k, &c, &sl);
+    const unsigned row_bytes = (unsigned)e.ns * (STORAGE == HSS_F32 ? 4u : 2u);
+    for (int r = 0; r < runs.n; ++r) {
+        const int beg = __builtin_amdgcn_readfirstlane(runs.start[r]);
+        const int end = __builtin_amdgcn_readfirstlane(runs.start[r + 1]);
+        const float h = uniform_f(runs.h[r]);
+        const OctTrace ot = oct_trace<FASTIDX>(h, 0.0f, e.h0);
+        const OctMid om = oct_mid<FASTIDX>(ot, oc, e.m0);
+        const OctKept kept = oct_kept_range(runs, beg, end, om, e.apm, active);
+        if (__builtin_amdgcn_ballot_w64(kept.lo < kept.hi) == 0) continue;
+        const OctTime otm = oct_time_terms<FASTIDX>(ot, oc, e.m0, om);
+        const OctDualTerms q = oct_dual_terms(h, e.h0, t0, e.m0, c, sl);
+        const int hi = otm.bad ? kept.lo : kept.hi;
+        const int steps = wave_max_steps(hi - kept.lo, end - beg);
+        for (int step = 0; step < steps; ++step) {
+            const int j = min(kept.lo + step, end - 1);
+            const OctRunTrace tr = runs.trace[j];
+            const float t = otm.th + otm.ah * (tr.m - om.mh);
+            int first;
+            float f;
+            const bool in = window_index<FASTIDX>(t, e.dt, e.inv_dt, e.ib, e.tau, &first, &f);
+            if (!(in & (kept.lo + step < hi))) continue;
+            float gi[D];
+            const Dual<2> tt = oct_time_from_terms(q, tr.m);
 #pragma unroll
-    for (int m = 0; m < D; ++m) gr[m] = 0.0f;
-    if (used > 0 && den > 0.0f) {
-        float num = 0.0f, lin = 0.0f;
+            for (int m = 0; m < D; ++m) gi[m] = (q.err == kNoError ? tt.d[m] : 0.0f) * e.inv_dt;
+            float y[N + 1];
+            const uint32_t row = __umul24((unsigned)tr.ti, row_bytes);
+            if constexpr (STORAGE == HSS_F32) {
+                const float *p = (const float *)at_bytes(e.samples, row + 4u * (uint32_t)first);
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            if (W == 0 && j >= e.w) continue;
-            num = __builtin_fmaf(A[j], A[j], num);
-            lin += A[j];
-        }
-        const float uden = (float)used * den;
-        sem = num / uden;
-        stk = lin / (float)(used * (unsigned)e.w);
-        const float scl = 2.0f / uden;
+                for (int j2 = 0; j2 <= N; ++j2) y[j2] = W > 0 || j2 <= e.w ? p[j2] : 0.0f;
+            } else {
+                const float sc = runs.scale[j];
+                const uint32_t at = (row >> 1) + (uint32_t)first;
+                if constexpr (W > 0) {
+                    read16<STORAGE, W>((const uint32_t *)e.samples, 0u, at, y);
 #pragma unroll
-        for (int m = 0; m < D; ++m) {
-            float a = 0.0f;
+                    for (int j2 = 0; j2 <= N; ++j2) y[j2] = y[j2] * sc;
+                } else {
+                    using Reader = SampleReader<STORAGE>;
+                    const Reader rd{(decltype(Reader::p))e.samples};
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                if (W == 0 && j >= e.w) continue;
-                a = __builtin_fmaf(A[j], G[j][m], a);
+                    for (int j2 = 0; j2 <= N; ++j2)
+                        y[j2] = j2 <= e.w ? rd((size_t)at + j2) * sc : 0.0f;
+                }
             }
-            gr[m] = scl * (a - sem * (float)used * H[m]);
+            sums.add(y, f, gi, e.w);
         }
     }
-    *S = sem;
-    *stack = stk;
-#pragma unroll
-    for (int m = 0; m < D; ++m) grad[m] = gr[m];
+    sums.reduce(e.w, S, stack, grad);
 }
 
 // ---------------------------------------------------------------------------
-// Kernels: one wave per (midpoint, 64 t0 samples); lane = t0 sample with its own point.
+// Kernels: one wave per (midpoint, 64 t0 samples); lane = t0 sample with its own point.  A
+// workgroup is one wave, for OCT four waves on neighbouring tiles of one midpoint, which
+// share the midpoint's offset runs in LDS.
 struct AdjointArgs {
     EvalCtx e;
     const int *mbeg;
@@ -375,7 +468,50 @@ struct AdjointArgs {
     int steps;            // polish steps
 };
 
-constexpr int kAdjThreads = kWave;
+template <int MODEL>
+constexpr int adj_waves() { return MODEL == HSS_OCT ? 4 : 1; }
+
+// Where a wave of an adjoint kernel works, and its evaluation of the gradient there.
+template <int MODEL, int W, int STORAGE>
+struct AdjointWave {
+    EvalCtx e;
+    int g, s, ns;
+    bool by_runs;
+    const OctRuns *runs;
+
+    // false: the workgroup has nothing to do.
+    __device__ __forceinline__ bool init(const AdjointArgs &a) {
+        constexpr int AW = adj_waves<MODEL>();
+        const int blk = logical_block(blockIdx.x, gridDim.x);
+        const int wg_per_mid = (a.ntiles + AW - 1) / AW;
+        const int slot = blk / wg_per_mid;
+        const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+        const int tile = (blk - slot * wg_per_mid) * AW + wave;
+        g = launch_midpoint(a.morder, a.nmid, slot);
+        if (g < 0) return false;
+        s = tile * kWave + ((int)threadIdx.x & (kWave - 1));  // (past ns: no active lane)
+        ns = a.e.ns;
+        e = midpoint_ctx(a.e, a.mbeg, a.mcnt, a.mm0, g);
+        by_runs = false;
+        if constexpr (MODEL == HSS_OCT) {
+            __shared__ OctRuns shared_runs;
+            by_runs = load_oct_runs(e, STORAGE == HSS_F32 ? 4 : 2, shared_runs);
+            runs = &shared_runs;
+        }
+        return true;
+    }
+
+    __device__ __forceinline__ void evaluate(float t0, const Candidate &k, bool active, float *S,
+                                             float *stack, float *grad) const {
+        if constexpr (MODEL == HSS_OCT) {
+            if (by_runs) {
+                evaluate_grad_runs<W, STORAGE>(e, *runs, t0, k, active, S, stack, grad);
+                return;
+            }
+        }
+        evaluate_grad<MODEL, W, STORAGE>(e, t0, t0 * t0, k, active, S, stack, grad);
+    }
+};
 
 template <int MODEL>
 __device__ __forceinline__ Candidate candidate_from_v(const float *p) {
@@ -393,19 +529,14 @@ __device__ __forceinline__ void grad_to_v(const float *p, float *g) {
 }
 
 template <int MODEL, int W, int STORAGE>
-__global__ __launch_bounds__(kAdjThreads) void gradient_kernel(AdjointArgs a) {
+__global__ __launch_bounds__(adj_waves<MODEL>() * kWave) void gradient_kernel(AdjointArgs a) {
     constexpr int D = model_np<MODEL>();
-    const int lane = threadIdx.x;
-    const int blk = logical_block(blockIdx.x, gridDim.x);
-    const int slot = blk / a.ntiles;
-    const int tile = blk - slot * a.ntiles;
-    const int g = launch_midpoint(a.morder, a.nmid, slot);
-    if (g < 0) return;
-    const int s = tile * kWave + lane;
-    const int ns = a.e.ns;
+    AdjointWave<MODEL, W, STORAGE> wv;
+    if (!wv.init(a)) return;
+    const int g = wv.g, s = wv.s, ns = wv.ns;
+    const EvalCtx &e = wv.e;
     const bool active = s < ns;
     const int sc = active ? s : 0;
-    const EvalCtx e = midpoint_ctx(a.e, a.mbeg, a.mcnt, a.mm0, g);
     const float *row = a.points + (size_t)g * (2 + D) * ns;
     float p[D];
 #pragma unroll
@@ -414,7 +545,7 @@ __global__ __launch_bounds__(kAdjThreads) void gradient_kernel(AdjointArgs a) {
     if (!(p[0] > 0.0f)) p[0] = 1.0f;
     const float t0 = (float)sc * e.dt;
     float S, stk, gr[D];
-    evaluate_grad<MODEL, W, STORAGE>(e, t0, t0 * t0, candidate_from_v<MODEL>(p), ok, &S, &stk, gr);
+    wv.evaluate(t0, candidate_from_v<MODEL>(p), ok, &S, &stk, gr);
     grad_to_v<MODEL>(p, gr);
     if (!active) return;
     float *out = a.out + (size_t)g * (2 + D) * ns;
@@ -431,19 +562,14 @@ __global__ __launch_bounds__(kAdjThreads) void gradient_kernel(AdjointArgs a) {
 // kept when S increases (mu /= 3), rejected otherwise (mu *= 4); mu starts at |dS/dx|^2.
 // S never decreases; the point stays in the box.
 template <int MODEL, int W, int STORAGE>
-__global__ __launch_bounds__(kAdjThreads) void polish_kernel(AdjointArgs a) {
+__global__ __launch_bounds__(adj_waves<MODEL>() * kWave) void polish_kernel(AdjointArgs a) {
     constexpr int D = model_np<MODEL>();
-    const int lane = threadIdx.x;
-    const int blk = logical_block(blockIdx.x, gridDim.x);
-    const int slot = blk / a.ntiles;
-    const int tile = blk - slot * a.ntiles;
-    const int g = launch_midpoint(a.morder, a.nmid, slot);
-    if (g < 0) return;
-    const int s = tile * kWave + lane;
-    const int ns = a.e.ns;
+    AdjointWave<MODEL, W, STORAGE> wv;
+    if (!wv.init(a)) return;
+    const int g = wv.g, s = wv.s, ns = wv.ns;
+    const EvalCtx &e = wv.e;
     const bool active = s < ns;
     const int sc = active ? s : 0;
-    const EvalCtx e = midpoint_ctx(a.e, a.mbeg, a.mcnt, a.mm0, g);
     const float *row = a.points + (size_t)g * (2 + D) * ns;
     float p[D], span[D];
 #pragma unroll
@@ -452,9 +578,8 @@ __global__ __launch_bounds__(kAdjThreads) void polish_kernel(AdjointArgs a) {
         p[m] = fminf(fmaxf(row[(2 + m) * ns + sc], a.lo[m]), a.hi[m]);
     }
     const float t0 = (float)sc * e.dt;
-    const float t0sq = t0 * t0;
     float S, stk, gr[D];
-    evaluate_grad<MODEL, W, STORAGE>(e, t0, t0sq, candidate_from_v<MODEL>(p), active, &S, &stk, gr);
+    wv.evaluate(t0, candidate_from_v<MODEL>(p), active, &S, &stk, gr);
     grad_to_v<MODEL>(p, gr);
     float mu = -1.0f;
     for (int it = 0; it < a.steps; ++it) {
@@ -474,8 +599,7 @@ __global__ __launch_bounds__(kAdjThreads) void polish_kernel(AdjointArgs a) {
             q[m] = fminf(fmaxf(p[m] + dx * span[m], a.lo[m]), a.hi[m]);
         }
         float S2, stk2, gr2[D];
-        evaluate_grad<MODEL, W, STORAGE>(e, t0, t0sq, candidate_from_v<MODEL>(q), live, &S2, &stk2,
-                                         gr2);
+        wv.evaluate(t0, candidate_from_v<MODEL>(q), live, &S2, &stk2, gr2);
         grad_to_v<MODEL>(q, gr2);
         if (live && S2 > S) {
             S = S2;
@@ -500,7 +624,8 @@ __global__ __launch_bounds__(kAdjThreads) void polish_kernel(AdjointArgs a) {
 
 template <int MODEL>
 int launch_adjoint(const AdjointArgs &a, int n_mid, int storage, bool polish, hipStream_t stream) {
-    const unsigned blocks = (unsigned)n_mid * (unsigned)a.ntiles;
+    constexpr int AW = adj_waves<MODEL>(), kAdjThreads = AW * kWave;
+    const unsigned blocks = (unsigned)n_mid * (unsigned)((a.ntiles + AW - 1) / AW);
     if (blocks == 0) return HSS_OK;
     int rc = dispatch_storage(storage, [&](auto S) {
         dispatch_window(a.e.w, fast_index_verified(a.e.dt, a.e.tau, stream), [&](auto Wc) {
