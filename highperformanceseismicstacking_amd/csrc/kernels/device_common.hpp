@@ -87,9 +87,10 @@ __device__ __forceinline__ float sqrt_of(float x) {
     else return sqrtf(x);
 }
 
+// oct_displacement: the same without the midpoint it is added to, *mh = m0 + d.
 template <bool FAST = false>
-__device__ __forceinline__ int oct_displaced_midpoint(float h, float h0, float t0, float m0,
-                                                      float c, float slope, float *mh) {
+__device__ __forceinline__ int oct_displacement(float h, float h0, float t0, float c, float slope,
+                                                float *d) {
     float theta = t0 * slope;
     float gamma = 2.0f * sqrt_of<FAST>(h * h + h0 * h0);
     float tn0_sq = t0 * t0 - c * h0 * h0;
@@ -101,8 +102,17 @@ __device__ __forceinline__ int oct_displaced_midpoint(float h, float h0, float t
     if (arg < 0) return kNegativeSquaredRoot;
     arg = theta_sq * gamma_sq + 2.0f * tn0_quad + 2.0f * sqrt_of<FAST>(arg);
     if (arg == 0) return kDivisionByZero;
-    *mh = m0 + 2.0f * theta * (h * h - h0 * h0) / sqrt_of<FAST>(arg);
+    *d = 2.0f * theta * (h * h - h0 * h0) / sqrt_of<FAST>(arg);
     return kNoError;
+}
+
+template <bool FAST = false>
+__device__ __forceinline__ int oct_displaced_midpoint(float h, float h0, float t0, float m0,
+                                                      float c, float slope, float *mh) {
+    float d;
+    const int err = oct_displacement<FAST>(h, h0, t0, c, slope, &d);
+    if (err == kNoError) *mh = m0 + d;
+    return err;
 }
 
 // OCT traveltime along the trajectory (reference: oct/common.cuh:37-94).

@@ -11,14 +11,16 @@
 //            stretch-free:  the (v, slope) picked at that very t0 (oct/stretch_free.cu:99-138);
 //            DE:            the start population of that t0 (oct/differential_evolution.cu:130-168).
 //
-// Each thread owns one (trace, midpoint); a workgroup's threads share the midpoint, which
-// the OCT path uses to take each candidate once per workgroup (select_oct).  For OCT a
-// trace whose midpoint distance exceeds apm + sqrt(h^2 + h0^2) cannot pass for any
+// CMP and ZO-CRS: each thread owns one (trace, midpoint).
+//
+// For OCT a trace whose midpoint distance exceeds apm + sqrt(h^2 + h0^2) cannot pass for any
 // candidate: the displaced midpoint
 // satisfies |mh - m0| = 2|theta||h^2-h0^2| / sqrt(theta^2 gamma^2 + 2q + 2sqrt(...))
 // <= |h^2-h0^2| / sqrt(h^2+h0^2) <= sqrt(h^2+h0^2), because the denominator is at least
 // |theta| gamma = 2|theta| sqrt(h^2+h0^2).  The test keeps a wide rounding margin, so it
 // only skips traces whose answer is certain.
+#include <algorithm>
+
 #include "de_impl.hpp"
 
 namespace hss {
@@ -30,6 +32,7 @@ struct SelectArgs {
     int ns;
     float dt;
     const float *m0;
+    int n;
     float apm, h0;
     int model;
     hss_oct_candidates oct;
@@ -46,9 +49,6 @@ __device__ __forceinline__ bool oct_within_reach(float m, float h, float m0, flo
     const float margin = 1e-4f * (fabsf(m0) + fabsf(m) + reach + apm) + 1e-3f;
     return fabsf(m - m0) <= apm + reach + margin;
 }
-
-// Distinct half offsets whose displaced midpoints a workgroup shares (16 KB of LDS).
-constexpr int kSelectOffsets = 16;
 
 // Candidates per t0 sample of one midpoint, in each mode.
 __device__ __forceinline__ int oct_candidates_per_sample(const SelectArgs &a) {
@@ -78,106 +78,132 @@ __device__ __forceinline__ void oct_candidate(const SelectArgs &a, int g, int s,
     }
 }
 
-// OCT: the candidates of a midpoint are the same for every trace, and a workgroup serves
-// one midpoint, so it takes each (t0 sample, candidate) pair once -- kSelectThreads at a
-// time (drawn, for DE start populations) -- and every thread whose trace is still open
-// tests them.  The displaced midpoint depends on the trace's half offset, not on its
-// midpoint, so when the workgroup's traces have at most kSelectOffsets distinct offsets
-// (their bit patterns) it is computed once per (offset, candidate) into a table, an
-// error stored as NaN (which fails the aperture test as the error does), and each thread
-// only compares its midpoint with its offset's row.  The mask is the OR over all
-// candidates, so neither the order nor the early exit changes it; the workgroup stops
-// when no trace is open.  Every thread takes part in the barriers (those past the last
-// trace have nothing open).
-__device__ void select_oct(const SelectArgs &a, int i, int g) {
-    __shared__ float cand_c[kSelectThreads], cand_s[kSelectThreads];
-    __shared__ float mh_tab[kSelectOffsets][kSelectThreads];
-    __shared__ uint32_t hbits[kSelectThreads];
-    __shared__ float off_h[kSelectOffsets];
-    __shared__ int slot_of[kSelectThreads];
-    __shared__ int row_open[kSelectOffsets];
-    __shared__ int n_off;
+// OCT.  What a candidate at a t0 does to a trace, mh = m0 + d, depends on the trace's half
+// offset alone through the displacement d, and |m - mh| <= apm rounds monotonically in d: the
+// displacements a trace accepts are an interval.  A workgroup takes a block of traces, a
+// group of midpoints with the same candidates (pairs: many midpoints; the other modes: one)
+// and a slice of the (t0, candidate) list.  It lists the block's distinct half offsets
+// (rows), works out each displacement of the slice once per row, and keeps for each row
+// kBins/rows bins over [-sqrt(h^2+h0^2), +sqrt(h^2+h0^2)], each with the smallest and largest
+// displacement in it.  A trace then looks at the few bins its interval reaches: the exact
+// test at a bin's two ends answers for the whole bin unless the interval lies strictly
+// between them (an aperture narrower than a bin), where the trace tests the slice itself.
+// The slices only ever set mask bytes that a first launch cleared, so they need not know of
+// each other.
+//
+// The masks are those of testing every (trace, midpoint, t0, candidate) one by one, at one
+// displacement per (t0, candidate, offset of the block) in place of one per midpoint and
+// 256-trace workgroup.  What bounds it is VALU work on the displacements (three square roots
+// and a division each).  Measured, 30 midpoints x 4832 traces, 1024 pairs at 1251 t0: 161 ->
+// 0.31 ms; 60 midpoints with start populations of 48: 7.8 -> 0.49 ms.  About as much time
+// again as the displacements take goes into the slices' looks at the traces: 256 workgroups of
+// 1024 threads measured 0.31 ms, 1024 of 256 threads, which look four times as often, 0.64.
+//
+// A block with more than kRowsMax offsets goes through them kRowsMax at a time, and one with
+// more than kOffsetsMax (offsets that hardly repeat) tests trace by trace, each candidate
+// drawn once per workgroup.
+constexpr int kRowsMax = 64;
+constexpr int kBins = 4096;
+constexpr int kOffsetsMax = 1024;
+constexpr int kSlots = 2 * kOffsetsMax;  // open-addressed table of the block's offsets
+constexpr int kOctThreads = 1024;
+constexpr int kTracesPerThread = 4;
+constexpr int kBlockTraces = kOctThreads * kTracesPerThread;
+constexpr int kPairMidpoints = 64;       // midpoints of a group in pairs mode
+
+// Floats as unsigned integers of the same order.
+__device__ __forceinline__ uint32_t order_key(float x) {
+    const uint32_t b = __float_as_uint(x);
+    return b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
+}
+__device__ __forceinline__ float order_value(uint32_t k) {
+    return __uint_as_float(k ^ ((k >> 31) ? 0x80000000u : 0xffffffffu));
+}
+
+struct OctRows {
+    unsigned long long slot[kSlots];  // 1 << 32 | the offset's bits; 0: empty
+    int number[kSlots];  // the offset's number; row = number - the pass's first
+    float h[kOffsetsMax];
+    float low[kRowsMax], per_unit[kRowsMax];  // the bins' start and bins per unit of d
+    uint32_t least[kBins], most[kBins];       // order keys; least > most: empty
+    unsigned long long filled[kBins / 64];    // bit b of word w: bin 64*w + b is not empty
+    int n;
+};
+
+__device__ __forceinline__ int offset_slot(const OctRows &t, uint32_t bits) {
+    int k = (int)((bits * 0x9e3779b1u) >> 16) % kSlots;
+    while (t.slot[k] != ((1ull << 32) | bits)) k = (k + 1) % kSlots;
+    return k;
+}
+
+__device__ __forceinline__ int bin_of(float d, float low, float per_unit, int nbins) {
+    return (int)fminf(fmaxf((d - low) * per_unit, 0.0f), (float)(nbins - 1));
+}
+
+// The exact test, by the side a displacement misses on: 0 inside the aperture, +1 too far
+// down (m - mh > apm), -1 too far up, 2 for a NaN.
+__device__ __forceinline__ int oct_side(float m, float m0, float d, float apm) {
+    const float x = m - (m0 + d);
+    if (fabsf(x) <= apm) return 0;
+    return x > apm ? 1 : (x < -apm ? -1 : 2);
+}
+
+// Whether some displacement of the slice [qa, qb) passes, one by one.
+__device__ bool oct_test_slice(const SelectArgs &a, int g, float m, float h, float m0, int NP,
+                               long long qa, long long qb) {
+    int s = (int)(qa / NP), p = (int)(qa - (long long)s * NP);
+    for (long long q = qa; q < qb; ++q) {
+        float c, slope, d;
+        oct_candidate(a, g, s, p, &c, &slope);
+        if (oct_displacement(h, a.h0, (float)s * a.dt, c, slope, &d) == kNoError &&
+            oct_side(m, m0, d, a.apm) == 0)
+            return true;
+        if (++p == NP) {
+            p = 0;
+            ++s;
+        }
+    }
+    return false;
+}
+
+// Every trace of the block tests the slice's candidates, kOctThreads of them at a time, which
+// the workgroup's threads draw into LDS; a midpoint is done when no trace is open.
+__device__ void select_oct_one_by_one(const SelectArgs &a, int i0, int g0, int g1,
+                                      unsigned reached, int NP, long long qa, long long qb,
+                                      uint32_t *cand_c, uint32_t *cand_s) {
     const int tid = (int)threadIdx.x;
-    const bool live = i < a.ntr;
-    const float m0 = a.m0[g];
-    const float m = live ? a.mid[i] : 0.0f;
-    const float h = live ? a.hoff[i] : 0.0f;
-    bool open = live && oct_within_reach(m, h, m0, a.h0, a.apm);
-    unsigned char used = 0;
-
-    // the workgroup's distinct offsets: the lowest live thread of each bit pattern takes a
-    // table row (in any order: the row numbers change nothing)
-    if (tid == 0) n_off = 0;
-    hbits[tid] = __float_as_uint(h);
-    slot_of[tid] = -1;
-    __syncthreads();
-    const int nlive = min(kSelectThreads, a.ntr - (int)(blockIdx.x * blockDim.x));
-    bool first = live;
-    for (int t = 0; first && t < tid; ++t) first = hbits[t] != hbits[tid];
-    if (first) {
-        const int r = atomicAdd(&n_off, 1);
-        slot_of[tid] = r;
-        if (r < kSelectOffsets) off_h[r] = h;
-    }
-    __syncthreads();
-    const bool tabled = n_off <= kSelectOffsets;  // (uniform)
-    int my_row = -1;
-    if (tabled && live) {
-        for (int t = 0; t < nlive; ++t)
-            if (hbits[t] == hbits[tid]) {
-                my_row = slot_of[t];
-                break;
-            }
-    }
-
-    const int NP = oct_candidates_per_sample(a);  // candidates per t0 sample
-    const long long total = (long long)a.ns * NP;
-    for (long long q0 = 0; q0 < total; q0 += kSelectThreads) {
-        if (!__syncthreads_or(open)) break;  // (also the barrier before LDS is rewritten)
-        if (tabled) {
-            // only the offsets some open trace still has get their row computed
-            if (tid < kSelectOffsets) row_open[tid] = 0;
-            __syncthreads();
-            if (open) row_open[my_row] = 1;
-            __syncthreads();
+    for (int g = g0; g < g1; ++g) {
+        const float m0 = a.m0[g];
+        unsigned open = 0;
+        for (int j = 0; j < kTracesPerThread; ++j) {
+            const int i = i0 + j * kOctThreads + tid;
+            if (((reached >> j) & 1) && oct_within_reach(a.mid[i], a.hoff[i], m0, a.h0, a.apm))
+                open |= 1u << j;
         }
-        const long long q = q0 + tid;
-        if (q < total) {
-            const int s = (int)(q / NP), p = (int)(q - (long long)s * NP);
-            float c, slope;
-            oct_candidate(a, g, s, p, &c, &slope);
-            if (tabled) {
-                const float t0 = (float)s * a.dt;
-                for (int row = 0; row < n_off; ++row) {
-                    if (!row_open[row]) continue;
-                    float mh;
-                    const int err = oct_displaced_midpoint(off_h[row], a.h0, t0, m0, c, slope, &mh);
-                    mh_tab[row][tid] = err == kNoError ? mh : __int_as_float(0x7fc00000);
-                }
-            } else {
-                cand_c[tid] = c;
-                cand_s[tid] = slope;
+        for (long long q0 = qa; q0 < qb; q0 += kOctThreads) {
+            if (!__syncthreads_or(open != 0)) break;  // (also before LDS is written again)
+            const long long q = q0 + tid;
+            if (q < qb) {
+                const int s = (int)(q / NP), p = (int)(q - (long long)s * NP);
+                float c, slope;
+                oct_candidate(a, g, s, p, &c, &slope);
+                cand_c[tid] = __float_as_uint(c);
+                cand_s[tid] = __float_as_uint(slope);
             }
-        }
-        __syncthreads();
-        if (open) {
-            const int n = (int)min((long long)kSelectThreads, total - q0);
-            if (tabled) {
-                for (int j = 0; j < n; ++j)
-                    if (fabsf(m - mh_tab[my_row][j]) <= a.apm) {
-                        used = 1;
-                        open = false;
-                        break;
-                    }
-            } else {
+            __syncthreads();
+            const int n = (int)min((long long)kOctThreads, qb - q0);
+            for (int j = 0; j < kTracesPerThread; ++j) {
+                if (!((open >> j) & 1)) continue;
+                const int i = i0 + j * kOctThreads + tid;
+                const float m = a.mid[i], h = a.hoff[i];
                 int s = (int)(q0 / NP), p = (int)(q0 - (long long)s * NP);
-                for (int j = 0; j < n; ++j) {
-                    float mh;
-                    const int err = oct_displaced_midpoint(h, a.h0, (float)s * a.dt, m0, cand_c[j],
-                                                           cand_s[j], &mh);
-                    if (err == kNoError && fabsf(m - mh) <= a.apm) {
-                        used = 1;
-                        open = false;
+                for (int k = 0; k < n; ++k) {
+                    float d;
+                    if (oct_displacement(h, a.h0, (float)s * a.dt, __uint_as_float(cand_c[k]),
+                                         __uint_as_float(cand_s[k]), &d) == kNoError &&
+                        oct_side(m, m0, d, a.apm) == 0) {
+                        a.mask[(size_t)g * a.ntr + i] = 1;
+                        open &= ~(1u << j);
                         break;
                     }
                     if (++p == NP) {
@@ -187,17 +213,164 @@ __device__ void select_oct(const SelectArgs &a, int i, int g) {
                 }
             }
         }
+        __syncthreads();  // before the next midpoint's candidates
     }
-    if (live) a.mask[(size_t)g * a.ntr + i] = used;
+}
+
+__global__ __launch_bounds__(kOctThreads) void select_oct_kernel(SelectArgs a, int group,
+                                                                    int slices) {
+    __shared__ OctRows t;
+    __shared__ int overflow;
+    const int tid = (int)threadIdx.x;
+    const int i0 = (int)blockIdx.x * kBlockTraces;
+    const int i1 = min(a.ntr, i0 + kBlockTraces);
+    const int g0 = (int)blockIdx.y * group, g1 = min(a.n, g0 + group);
+    const int NP = oct_candidates_per_sample(a);
+    const long long total = (long long)a.ns * NP;
+    const long long qa = total * (int)blockIdx.z / slices;
+    const long long qb = total * ((int)blockIdx.z + 1) / slices;
+    if (qa >= qb) return;  // (uniform)
+
+    // the distinct offsets of the block's traces that some midpoint of the group can reach
+    for (int k = tid; k < kSlots; k += kOctThreads) t.slot[k] = 0;
+    if (tid == 0) overflow = 0;
+    __syncthreads();
+    unsigned reached = 0;  // bit j: trace i0 + kOctThreads*j + tid
+    for (int j = 0; j < kTracesPerThread; ++j) {
+        const int i = i0 + j * kOctThreads + tid;
+        if (i >= i1) break;
+        const float m = a.mid[i], h = a.hoff[i];
+        bool any = false;
+        for (int g = g0; g < g1 && !any; ++g) any = oct_within_reach(m, h, a.m0[g], a.h0, a.apm);
+        if (!any) continue;
+        reached |= 1u << j;
+        const unsigned long long key = (1ull << 32) | __float_as_uint(h);
+        int k = (int)((__float_as_uint(h) * 0x9e3779b1u) >> 16) % kSlots;
+        int tries = 0;
+        for (; tries < kSlots; ++tries, k = (k + 1) % kSlots) {
+            const unsigned long long was = atomicCAS(&t.slot[k], 0ull, key);
+            if (was == 0ull || was == key) break;
+        }
+        if (tries == kSlots) overflow = 1;
+    }
+    __syncthreads();
+    if (tid < kWave) {  // number the used slots
+        int n = 0;
+        for (int k0 = 0; k0 < kSlots; k0 += kWave) {
+            const unsigned long long key = t.slot[k0 + tid];
+            const unsigned long long used = __builtin_amdgcn_ballot_w64(key != 0);
+            const int number = n + __builtin_popcountll(used & ((1ull << tid) - 1));
+            t.number[k0 + tid] = number;
+            if (key != 0 && number < kOffsetsMax) t.h[number] = __uint_as_float((uint32_t)key);
+            n += __builtin_popcountll(used);
+        }
+        if (tid == 0) {
+            t.n = n;
+            if (n > kOffsetsMax) overflow = 1;
+        }
+    }
+    __syncthreads();
+    const int offsets = t.n;
+    if (offsets == 0) return;  // (uniform, as `overflow` is)
+    if (overflow) {
+        select_oct_one_by_one(a, i0, g0, g1, reached, NP, qa, qb, t.least, t.most);
+        return;
+    }
+    const int passes = (offsets + kRowsMax - 1) / kRowsMax;
+    const int per_pass = (offsets + passes - 1) / passes;
+    const int nbins = per_pass <= kRowsMax / 4 ? kBins / (kRowsMax / 4) : kBins / kRowsMax;
+    for (int first = 0; first < offsets; first += per_pass) {
+        const int rows = min(per_pass, offsets - first);
+        for (int k = tid; k < kBins; k += kOctThreads) {
+            t.least[k] = 0xffffffffu;
+            t.most[k] = 0;
+        }
+        if (tid < rows) {
+            const float h = t.h[first + tid];
+            const float r = sqrtf(h * h + a.h0 * a.h0);
+            t.low[tid] = -r;
+            t.per_unit[tid] = r > 0.0f && r < INFINITY ? (float)nbins / (2.0f * r) : 0.0f;
+        }
+        __syncthreads();
+
+        // the slice's displacements, each thread its own candidates
+        for (long long q = qa + tid; q < qb; q += kOctThreads) {
+            const int s = (int)(q / NP), p = (int)(q - (long long)s * NP);
+            float c, slope;
+            oct_candidate(a, g0, s, p, &c, &slope);
+            const float t0 = (float)s * a.dt;
+            for (int row = 0; row < rows; ++row) {
+                float d;
+                if (oct_displacement(t.h[first + row], a.h0, t0, c, slope, &d) != kNoError ||
+                    d != d)
+                    continue;
+                const int b = row * nbins + bin_of(d, t.low[row], t.per_unit[row], nbins);
+                const uint32_t key = order_key(d);
+                if (key < t.least[b]) atomicMin(&t.least[b], key);
+                if (key > t.most[b]) atomicMax(&t.most[b], key);
+            }
+        }
+        __syncthreads();
+        for (int k = tid; k < kBins; k += kOctThreads) {
+            const unsigned long long w = __builtin_amdgcn_ballot_w64(t.least[k] <= t.most[k]);
+            if ((k & 63) == 0) t.filled[k / 64] = w;
+        }
+        __syncthreads();
+
+        for (int j = 0; j < kTracesPerThread; ++j) {
+            if (!((reached >> j) & 1)) continue;
+            const int i = i0 + j * kOctThreads + tid;
+            const float m = a.mid[i], h = a.hoff[i];
+            const int row = t.number[offset_slot(t, __float_as_uint(h))] - first;
+            if (row < 0 || row >= rows) continue;
+            const float low = t.low[row], per_unit = t.per_unit[row];
+            for (int g = g0; g < g1; ++g) {
+                const float m0 = a.m0[g];
+                if (!oct_within_reach(m, h, m0, a.h0, a.apm)) continue;
+                // the bins of the accepted displacements, m - m0 -+ apm and a margin for
+                // rounding
+                const float margin = 1e-4f * (fabsf(m0) + fabsf(m) - low + a.apm) + 1e-3f;
+                const int ba = bin_of(m - m0 - a.apm - margin, low, per_unit, nbins);
+                const int bb = bin_of(m - m0 + a.apm + margin, low, per_unit, nbins);
+                bool used = false, unsure = false;
+                for (int b = ba; b <= bb && !used; ++b) {
+                    const int bin = row * nbins + b;
+                    const unsigned long long rest = t.filled[bin / 64] >> (bin & 63);
+                    if (rest == 0) {  // on to the next word
+                        b += 63 - (bin & 63);
+                        continue;
+                    }
+                    b += __builtin_ctzll(rest);
+                    if (b > bb) break;
+                    const int at = row * nbins + b;
+                    const int lo = oct_side(m, m0, order_value(t.least[at]), a.apm);
+                    const int hi = oct_side(m, m0, order_value(t.most[at]), a.apm);
+                    used = lo == 0 || hi == 0;
+                    unsure = unsure || lo != hi;
+                }
+                if (!used && unsure) used = oct_test_slice(a, g, m, h, m0, NP, qa, qb);
+                if (used) a.mask[(size_t)g * a.ntr + i] = 1;
+            }
+        }
+        __syncthreads();  // the bins are cleared next
+    }
+}
+
+__global__ __launch_bounds__(kSelectThreads) void clear_mask_kernel(unsigned char *mask,
+                                                                    unsigned long long bytes) {
+    const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
+    unsigned long long b = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+    // 16 bytes at a time from the first aligned address on
+    const unsigned long long head = min(bytes, (unsigned long long)(-(uintptr_t)mask & 15u));
+    const unsigned long long quads = (bytes - head) / 16;
+    if (b < head) mask[b] = 0;
+    if (b < bytes - head - quads * 16) mask[head + quads * 16 + b] = 0;
+    for (; b < quads; b += stride) ((uint4 *)(mask + head))[b] = uint4{0, 0, 0, 0};
 }
 
 __global__ __launch_bounds__(kSelectThreads) void select_traces_kernel(SelectArgs a) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int g = blockIdx.y;
-    if (a.model == HSS_OCT) {  // (uniform over the launch)
-        select_oct(a, i, g);
-        return;
-    }
     if (i >= a.ntr) return;
     const float m0 = a.m0[g];
     const float m = a.mid[i];
@@ -207,6 +380,34 @@ __global__ __launch_bounds__(kSelectThreads) void select_traces_kernel(SelectArg
     else  // HSS_ZOCRS
         used = fabsf(m0 - m) <= a.apm;
     a.mask[(size_t)g * a.ntr + i] = used;
+}
+
+// OCT: clear the masks, then set them.  About kSelectWorkgroups workgroups share the (t0,
+// candidate) list, slices of at least kSliceLeast (a slice costs its workgroup one look at
+// every trace of the block for every midpoint of the group).
+constexpr long long kSelectWorkgroups = 256, kSliceLeast = 1024;
+
+static int select_oct(const SelectArgs &a, hipStream_t stream) {
+    const unsigned long long bytes = (unsigned long long)a.n * (unsigned long long)a.ntr;
+    const unsigned clear = (unsigned)std::min<unsigned long long>(
+        (bytes / 16 + kSelectThreads) / kSelectThreads, 4096);
+    hipLaunchKernelGGL(clear_mask_kernel, dim3(clear), dim3(kSelectThreads), 0, stream, a.mask,
+                       bytes);
+    int rc = hip_status(hipGetLastError());
+    if (rc != HSS_OK) return rc;
+    const int group = a.oct.mode == HSS_OCT_PAIRS ? kPairMidpoints : 1;
+    const long long per_sample = a.oct.mode == HSS_OCT_PAIRS      ? a.oct.npairs
+                                 : a.oct.mode == HSS_OCT_DE_START ? a.oct.NP
+                                                                  : 1;
+    const long long total = (long long)a.ns * per_sample;
+    if (total == 0) return HSS_OK;
+    const long long x = ((long long)a.ntr + kBlockTraces - 1) / kBlockTraces;
+    const long long y = (a.n + group - 1) / group;
+    const long long slices =
+        std::max(1ll, std::min((kSelectWorkgroups + x * y - 1) / (x * y), total / kSliceLeast));
+    hipLaunchKernelGGL(select_oct_kernel, dim3((unsigned)x, (unsigned)y, (unsigned)slices),
+                       dim3(kOctThreads), 0, stream, a, group, (int)slices);
+    return hip_status(hipGetLastError());
 }
 
 }  // namespace hss
@@ -227,6 +428,7 @@ extern "C" int hss_select_traces(const hss_traces *traces, int model, int32_t n,
     a.ns = traces->ns;
     a.dt = traces->dt;
     a.m0 = d_m0;
+    a.n = n;
     a.apm = apm;
     a.h0 = h0;
     a.model = model;
@@ -248,6 +450,7 @@ extern "C" int hss_select_traces(const hss_traces *traces, int model, int32_t n,
         }
     }
     if (n == 0 || traces->ntr == 0) return HSS_OK;
+    if (model == HSS_OCT) return select_oct(a, (hipStream_t)stream);
     dim3 grid((traces->ntr + kSelectThreads - 1) / kSelectThreads, n);
     hipLaunchKernelGGL(select_traces_kernel, grid, dim3(kSelectThreads), 0, (hipStream_t)stream, a);
     return hip_status(hipGetLastError());
