@@ -6,6 +6,7 @@
 #include "kernels/adjoint.hpp"
 #include "kernels/de_impl.hpp"
 #include "kernels/grid_impl.hpp"
+#include "kernels/grid_spread.hpp"
 #include "kernels/grid_staged.hpp"
 #include "kernels/launch_util.hpp"
 #include "kernels/sf_impl.hpp"
@@ -203,6 +204,23 @@ int hss_grid_semblance(const hss_traces *traces, const hss_midpoints *mids, int 
             default: return launch_grid_oct(la, slots, variant, traces->storage, sh.cpl, st);
         }
     };
+    if (!grid_shape_pinned(model, traces->w, variant, traces->storage) &&
+        spread_wanted(model, traces->storage, (long long)mids->n * a.ntiles)) {
+        const int tl = spread_tl(model, mids->n, traces->ns, P);
+        int status = HSS_OK;
+        bool done;
+        switch (model) {
+            case HSS_CMP:
+                done = launch_spread_cmp(a, mids->n, variant, traces->storage, tl, st, &status);
+                break;
+            case HSS_ZOCRS:
+                done = launch_spread_zocrs(a, mids->n, variant, traces->storage, tl, st, &status);
+                break;
+            default:
+                done = launch_spread_oct(a, mids->n, variant, traces->storage, tl, st, &status);
+        }
+        if (done) return status;
+    }
     // timing runs must not add to the accumulating rejection counts
     GridArgs probe = a;
     probe.not_used = nullptr;

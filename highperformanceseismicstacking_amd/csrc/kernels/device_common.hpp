@@ -502,6 +502,13 @@ __device__ __forceinline__ float uniform_f(float x) {
     return __int_as_float(b);
 }
 
+// A wave-uniform value in a vector register: an operation with a scalar-register source
+// issues at half the rate of one on vector registers (window.hpp).
+__device__ __forceinline__ float vector_f(float x) {
+    __asm__("" : "+v"(x));
+    return x;
+}
+
 // threadIdx.x through an empty asm statement: what is derived from it at a point of use
 // (a lane's LDS slots, its output row, its sample) is recomputed there from the one
 // register that holds the thread index, instead of being kept in registers of its own (or

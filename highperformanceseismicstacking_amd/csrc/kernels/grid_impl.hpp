@@ -41,6 +41,7 @@ struct GridArgs {
     int ntiles;      // 64-sample t0 tiles of a midpoint
     int tt;          // t0 tiles per workgroup (1, 2 or 4; the waves split into tt x 4/tt)
     int wg_per_mid;  // workgroups per midpoint, ceil(ntiles / tt)
+    int tl;          // grid_spread.hpp: log2 of the t0 samples per workgroup
     float *result;
     float *sembl;
     float *stack;

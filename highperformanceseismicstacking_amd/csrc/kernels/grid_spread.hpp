@@ -1,0 +1,191 @@
+// Grid search spread over the chip: a workgroup takes T consecutive t0 samples (T a power of
+// two up to 64), and its 512 lanes split into 512/T candidate groups of two candidates per
+// lane and round.  Each lane keeps its running best; lanes that share a sample merge them as
+// the other grid kernels do (the larger value, then the lower index), so the results are the
+// same bits.
+//
+// The one-tile kernels give a midpoint of ns samples ns/64 workgroups, one 60-trace gather 16
+// of them on 256 CUs, and a workgroup of a large launch runs long enough to leave a tail.
+// With T down to 4 a gather fills the chip, and a line's launch ends evenly.  Candidates of
+// one lane group are neighbours, so windows stay close together where T is small.  Measured
+// (T in brackets; before -> here): one 60-trace gather, 256 candidates [4] 425 -> 51 us (the
+// staged kernel); ZO-CRS, 24 midpoints, BF16 [16] 119 -> 39.9 ms, 200 midpoints 97 -> 82 ms;
+// OCT, 30 midpoints, FP16 [16] 188 -> 76 ms, 250 midpoints [32] 204 -> 137 ms; OCT, 30
+// midpoints in the reference's order, EXACT 105 -> 74 ms.  What bounds it then is VALU issue:
+// the 16-bit lanes widen and scale every sample of their own windows, the price of not sharing
+// LDS segments.
+#pragma once
+
+#include "eval_lanes.hpp"
+#include "grid_impl.hpp"
+
+namespace hss {
+
+constexpr int kSpreadWaves = 8;
+constexpr int kSpreadThreads = kSpreadWaves * kWave;
+constexpr int kSpreadCpl = 2;
+// Register budget, as waves per SIMD (a workgroup is two of them).  Windows of up to 11 samples
+// of CMP and ZO-CRS fit six (39.9 against 42.8 ms at four, ZO-CRS, 24 midpoints); OCT, whose
+// terms would spill, and wider windows take four (OCT 76 ms, 79 at six; w = 15: 43 against 59
+// at two, which leaves one workgroup per CU).
+template <int MODEL, int W>
+constexpr int spread_min_waves() { return MODEL == HSS_OCT || W > 11 ? 4 : 6; }
+
+template <int MODEL, int W, int VARIANT, int STORAGE>
+__global__ __launch_bounds__(kSpreadThreads)
+__attribute__((amdgpu_waves_per_eu(spread_min_waves<MODEL, W>(), 8))) void grid_spread_kernel(GridArgs a) {
+    constexpr int NP = MODEL == HSS_CMP ? 1 : (MODEL == HSS_ZOCRS ? 3 : 2);
+    constexpr int CPL = kSpreadCpl;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int T = 1 << a.tl;  // t0 samples per workgroup
+    const int blk = logical_block(blockIdx.x, gridDim.x);
+    const int slot = blk / a.wg_per_mid;
+    const int g = launch_midpoint(a.morder, a.nmid, slot);
+    if (g < 0) return;  // (the whole workgroup)
+    const int s0 = (blk - slot * a.wg_per_mid) * T;
+    const int s = s0 + (lane & (T - 1));
+    const int ns = a.e.ns;
+    const bool active = s < ns;
+    const float t0 = (float)s * a.e.dt;
+    const EvalCtx e = midpoint_ctx(a.e, a.mbeg, a.mcnt, a.mm0, g);
+    const int per_wave = kWave >> a.tl, groups = kSpreadWaves * per_wave;
+    const int grp = wave * per_wave + (lane >> a.tl);
+
+    float best = -1.0f, bstack = 0.0f;
+    int bidx = -1;
+    unsigned long long rejected = 0;
+    bool by_runs = false;
+    if constexpr (MODEL == HSS_OCT) by_runs = oct_offset_runs_long(e);
+    for (int r0 = 0; r0 < a.P; r0 += groups * CPL) {
+        const int q0 = r0 + grp * CPL;
+        Candidate k[CPL];
+        bool on[CPL];
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            on[c] = q0 + c < a.P;
+            k[c] = load_candidate<MODEL>(a.params, min(q0 + c, a.P - 1));
+        }
+        float S[CPL], stk[CPL];
+        unsigned rej = 0;
+        evaluate_lanes<MODEL, W, VARIANT, STORAGE, CPL>(e, t0, t0 * t0, k, on, active, by_runs, S,
+                                                        stk, &rej);
+        rejected += rej;
+        if (!active) continue;
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            if (!on[c]) continue;
+            const int q = q0 + c;
+            if (a.sembl) a.sembl[((size_t)g * ns + s) * a.P + q] = S[c];
+            if (a.stack) a.stack[((size_t)g * ns + s) * a.P + q] = stk[c];
+            if (S[c] > best) {
+                best = S[c];
+                bstack = stk[c];
+                bidx = q;
+            }
+        }
+    }
+    if (MODEL == HSS_OCT && a.not_used) {
+        const unsigned long long tot = wave_sum_u64(rejected);
+        if (lane == 0 && tot) atomicAdd(a.not_used + g, tot);
+    }
+
+    // the best of the lanes that share a sample: the larger value, then the lower index
+    // (as merge_bests), first inside the wave, then over the waves
+    auto better = [&](float v, float st, int i) {
+        if (i >= 0 && (v > best || (v == best && i < bidx) || bidx < 0)) {
+            best = v;
+            bstack = st;
+            bidx = i;
+        }
+    };
+    for (int off = T; off < kWave; off <<= 1) {
+        const float v = __shfl_xor(best, off, kWave), st = __shfl_xor(bstack, off, kWave);
+        const int i = __shfl_xor(bidx, off, kWave);
+        better(v, st, i);
+    }
+    __shared__ float sh_best[kSpreadWaves][kWave], sh_stack[kSpreadWaves][kWave];
+    __shared__ int sh_idx[kSpreadWaves][kWave];
+    sh_best[wave][lane] = best;
+    sh_stack[wave][lane] = bstack;
+    sh_idx[wave][lane] = bidx;
+    __syncthreads();
+    if (wave != 0 || lane >= T || !active) return;
+#pragma unroll
+    for (int v = 1; v < kSpreadWaves; ++v) better(sh_best[v][lane], sh_stack[v][lane], sh_idx[v][lane]);
+    float *res = a.result + (size_t)g * (2 + NP) * ns;
+    res[s] = bidx >= 0 ? best : -1.0f;
+    res[ns + s] = bidx >= 0 ? bstack : 0.0f;
+    if (bidx >= 0) {
+        const Candidate k = load_candidate<MODEL>(a.params, bidx);
+        res[2 * ns + s] = 2 / sqrtf(k.c);
+        if constexpr (NP >= 2) res[3 * ns + s] = k.p1;
+        if constexpr (NP >= 3) res[4 * ns + s] = k.p2;
+    } else {
+#pragma unroll
+        for (int d = 0; d < NP; ++d) res[(2 + d) * ns + s] = 0.0f;
+    }
+}
+
+// log2 of T.  The workgroups should outnumber the CUs eight times, for a launch that ends
+// evenly; below that T halves down to 4.  T also stays at 1024/P or above, where one round
+// takes all P candidates (64 candidates on 12 midpoints: T = 16 190 us, T = 8, half of the
+// lanes idle, 270 us).  T = 16 is the largest that pays (ZO-CRS, 100 midpoints: 51/45/41.9/
+// 41.4 ms at 64/32/16/8), 32 for OCT (100 midpoints: 62/57.6/59.1/75 ms), whose runs visit
+// the traces that any of a wave's candidates keeps.
+constexpr int kSpreadWorkgroups = 2048;
+inline int spread_tl(int model, int n_slots, int ns, int P) {
+    int tl = model == HSS_OCT ? 5 : 4;
+    while (tl > 2 && (long long)n_slots * ((ns + (1 << tl) - 1) >> tl) < kSpreadWorkgroups) --tl;
+    while (tl < 6 && (2048ll >> tl) > P) ++tl;
+    return tl;
+}
+
+// Whether a launch takes this kernel when no shape is pinned for it: ZO-CRS and OCT always
+// (measured faster at every size, above), CMP below the size where the staged kernel, which
+// reads and widens a sample once for many windows, has enough workgroups (FP32, w = 11, 512
+// candidates: 288 workgroups of it 1.62 against 1.19 ms, 600 2.17 against 2.08, 1200 3.70
+// against 3.80; FP16, w = 15: 288 1.93 against 2.08, 1200 4.45 against 6.5).
+inline bool spread_wanted(int model, int storage, long long tiles) {
+    if (model != HSS_CMP) return true;
+    return tiles <= (storage == HSS_F32 ? 768 : 240);
+}
+
+// false: this window, variant or trace length has no such kernel.
+template <int MODEL>
+bool launch_grid_spread(const GridArgs &a, int n_slots, int variant, int storage, int tl,
+                        hipStream_t stream, int *status) {
+    if (variant == HSS_KAHAN || a.e.ns <= a.e.w ||
+        !fast_index_verified(a.e.dt, a.e.tau, stream))
+        return false;
+    GridArgs la = a;
+    la.tl = tl;
+    la.wg_per_mid = (a.e.ns + (1 << tl) - 1) >> tl;
+    const unsigned long long blocks = (unsigned long long)n_slots * la.wg_per_mid;
+    if (blocks == 0 || blocks > 0x7fffffffull) return false;
+    bool done = false;
+    const int rc = dispatch_storage(storage, [&](auto S) {
+        dispatch_variant(variant, [&](auto V) {
+            dispatch_window(a.e.w, true, [&](auto Wc) {
+                constexpr int WW = decltype(Wc)::value, VV = decltype(V)::value,
+                              SS = decltype(S)::value;
+                if constexpr (WW > 0 && VV != HSS_KAHAN) {
+                    hipLaunchKernelGGL((grid_spread_kernel<MODEL, WW, VV, SS>),
+                                       dim3((unsigned)blocks), dim3(kSpreadThreads), 0, stream, la);
+                    done = true;
+                }
+            });
+        });
+    });
+    *status = rc != HSS_OK ? rc : (done ? hip_status(hipGetLastError()) : HSS_OK);
+    return done;
+}
+
+bool launch_spread_cmp(const GridArgs &a, int n_slots, int variant, int storage, int tl,
+                       hipStream_t stream, int *status);
+bool launch_spread_zocrs(const GridArgs &a, int n_slots, int variant, int storage, int tl,
+                         hipStream_t stream, int *status);
+bool launch_spread_oct(const GridArgs &a, int n_slots, int variant, int storage, int tl,
+                       hipStream_t stream, int *status);
+
+}  // namespace hss

@@ -77,13 +77,6 @@ struct StagedTrace {
     uint32_t row;
 };
 
-// A wave-uniform value in a vector register: an operation with a scalar-register source
-// issues at half the rate of one on vector registers (window.hpp).
-__device__ __forceinline__ float vector_f(float x) {
-    __asm__("" : "+v"(x));
-    return x;
-}
-
 template <int W, int VARIANT, int STORAGE, int CPL>
 __global__ __launch_bounds__(kStagedThreads)
 __attribute__((amdgpu_waves_per_eu(staged_min_waves<W, VARIANT, CPL>(), 8))) void grid_staged_kernel(

@@ -54,6 +54,9 @@ struct GridShape {
     int staged;
 };
 
+// Whether hss_grid_set_shape holds a shape for this key on the current device.
+bool grid_shape_pinned(int model, int w, int variant, int storage);
+
 // The shape for this key, tuned on the first large launch by timing launch(shape, slots)
 // for each shape on the first `slots` launch slots of the batch (tune.hip).
 int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, int ntiles,

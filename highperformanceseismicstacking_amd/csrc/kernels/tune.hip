@@ -1,4 +1,6 @@
-// The launch-shape autotuner of the grid search.
+// The launch-shape autotuner of the grid search's one-tile kernels (large CMP launches, the
+// compensated variant, and windows without a compiled size; other launches take the spread
+// kernel, whose shape follows from the launch's size: grid_spread.hpp).
 //
 // Three knobs (grid_impl.hpp, grid_staged.hpp), none of which changes a result bit:
 //  * the parameter tile, candidates per lane (CPL = 1 or 2): two candidates share the
@@ -34,7 +36,11 @@ namespace hss {
 
 namespace {
 std::mutex tune_mu;
-std::map<std::tuple<int, int, int, int, int>, GridShape> tune_cache;
+struct TunedShape {
+    GridShape shape;
+    bool pinned;  // by hss_grid_set_shape
+};
+std::map<std::tuple<int, int, int, int, int>, TunedShape> tune_cache;
 
 bool tuning_enabled() {
     const char *v = std::getenv("HSS_AUTOTUNE");
@@ -65,7 +71,7 @@ int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, in
         std::lock_guard<std::mutex> lock(tune_mu);
         auto it = tune_cache.find(key);
         if (it != tune_cache.end()) {
-            *shape_out = it->second;
+            *shape_out = it->second.shape;
             return HSS_OK;
         }
     }
@@ -114,7 +120,7 @@ int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, in
     if (rc != HSS_OK) return rc;
     if (!timed) return HSS_OK;  // a HIP call failed: keep the default, cache nothing
     std::lock_guard<std::mutex> lock(tune_mu);
-    tune_cache[key] = best;
+    tune_cache[key] = TunedShape{best, false};
     *shape_out = best;
     return HSS_OK;
 }
@@ -125,13 +131,21 @@ void tuned_grid_store(int dev, int model, int w, int variant, int storage, GridS
     if (shape.cpl == 0)
         tune_cache.erase(key);
     else
-        tune_cache[key] = shape;
+        tune_cache[key] = TunedShape{shape, true};
 }
 
 GridShape tuned_grid_lookup(int dev, int model, int w, int variant, int storage) {
     std::lock_guard<std::mutex> lock(tune_mu);
     auto it = tune_cache.find(std::make_tuple(dev, model, w, variant, storage));
-    return it == tune_cache.end() ? GridShape{0, 0, 0} : it->second;
+    return it == tune_cache.end() ? GridShape{0, 0, 0} : it->second.shape;
+}
+
+bool grid_shape_pinned(int model, int w, int variant, int storage) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(tune_mu);
+    auto it = tune_cache.find(std::make_tuple(dev, model, w, variant, storage));
+    return it != tune_cache.end() && it->second.pinned;
 }
 
 }  // namespace hss

@@ -178,7 +178,12 @@ int hss_grid_semblance_plain(const hss_traces *traces, int model, const float *d
                              const int32_t *h_count, const float *h_m0, float h0, float apm,
                              float *d_sembl, float *d_stack, float *d_result, void *stream);
 
-/* The launch shape the grid-search autotuner chose on the current device for (model, w,
+/* Launch shapes of the grid search.  Unless a shape is pinned for the key (below), ZO-CRS and
+ * OCT launches and small CMP launches (up to 768 64-sample tiles over all midpoints, 240 with
+ * 16-bit storage) of a compiled window size and without compensation take a kernel whose
+ * shape follows from the launch's size, and tune nothing.
+ *
+ * The launch shape the grid-search autotuner chose on the current device for (model, w,
  * variant, storage): *cpl = candidates per lane (1 or 2), *t0_tiles = 64-sample t0 tiles
  * per workgroup (1, 2 or 4; the workgroup's four waves split into that many tiles times
  * 4 / t0_tiles candidate groups), *staged = 1 when the workgroup stages each trace's span
