@@ -184,9 +184,15 @@ __device__ __forceinline__ float sqrt_time(float x) {
     return r;
 }
 
+// (FAST without a shift: a negative radicand's root is a NaN or +inf, which no window accepts,
+// so its sign need not be tested.)
 template <bool FAST, bool SHIFT = false>
 __device__ __forceinline__ bool zocrs_time_from(float mid_part, float c_h2, float *t) {
     const float tmp = mid_part + c_h2;
+    if constexpr (FAST && !SHIFT) {
+        *t = sqrt_time<FAST, SHIFT>(tmp);
+        return true;
+    }
     if (tmp >= 0) {
         *t = sqrt_time<FAST, SHIFT>(tmp);
         return true;
@@ -398,8 +404,13 @@ __device__ __forceinline__ bool oct_traveltime_at(const OctMid &d, const OctTime
 //              hi = -2.
 // NaN fails both compares.  index_bounds() computes (lo, hi) on the host; ns < 2^24
 // keeps hi exact.
+// FAST (tau >= 1) makes the test on the index: tau <= k < K as one unsigned comparison,
+// k - tau < span = max(K - tau, 0), of a value the window's address needs anyway.  The
+// conversion gives 0 for a NaN and saturates, both outside; ZO-CRS differential evolution,
+// 32 midpoints, 92.6 -> 90.6 ms against the two float comparisons.
 struct IndexBounds {
     float lo, hi;
+    int tau, span;
 };
 
 __host__ __device__ inline IndexBounds index_bounds(int ns, int tau) {
@@ -407,6 +418,8 @@ __host__ __device__ inline IndexBounds index_bounds(int ns, int tau) {
     b.lo = tau == 0 ? -1.0f : __builtin_nextafterf((float)tau, 0.0f);
     const int K = ns - tau - 1;
     b.hi = K >= 1 ? (float)K : -2.0f;
+    b.tau = tau;
+    b.span = K > tau ? K - tau : 0;
     return b;
 }
 
@@ -436,6 +449,7 @@ __device__ __forceinline__ bool window_k(float t, float dt, float inv, IndexBoun
     if constexpr (FAST) *frac = __builtin_amdgcn_fractf(ti);
     else *frac = ti - (float)k;
     *k_out = k;
+    if constexpr (FAST) return (unsigned)(k - ib.tau) < (unsigned)ib.span;
     return ti > ib.lo && ti < ib.hi;
 }
 
