@@ -145,6 +145,41 @@ __device__ __forceinline__ Candidate de_candidate(const float *x) {
     return k;
 }
 
+// The end of a run for sample s of midpoint g: the first best individual, and the population.
+template <int D, class Rec>
+__device__ __forceinline__ void de_report(const DeArgs &a, int g, int s, const Rec &rec) {
+    const int ns = a.e.ns, NP = a.NP;
+    const int cur = (a.G - 1) & 1;
+    // selectBestIndividuals*: first strict maximum of S over the population
+    float best = -1.0f, bstack = 0.0f;
+    int bi = -1;
+    for (int i = 0; i < NP; ++i) {
+        const float S = *rec(cur, i, D);
+        if (S > best) {
+            best = S;
+            bstack = *rec(cur, i, D + 1);
+            bi = i;
+        }
+    }
+    float *res = a.result + (size_t)g * (2 + D) * ns;
+    res[s] = best;
+    res[ns + s] = bi >= 0 ? bstack : 0.0f;
+#pragma unroll
+    for (int d = 0; d < D; ++d) res[(2 + d) * ns + s] = bi >= 0 ? *rec(cur, bi, d) : 0.0f;
+    if (a.pop_x) {
+        for (int i = 0; i < NP; ++i)
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+                a.pop_x[(((size_t)g * ns + s) * NP + i) * D + d] = *rec(cur, i, d);
+    }
+    if (a.pop_fx) {
+        for (int i = 0; i < NP; ++i) {
+            a.pop_fx[(((size_t)g * ns + s) * NP + i) * 2] = *rec(cur, i, D);
+            a.pop_fx[(((size_t)g * ns + s) * NP + i) * 2 + 1] = *rec(cur, i, D + 1);
+        }
+    }
+}
+
 template <int MODEL, int W, int VARIANT, int STORAGE>
 __global__ __launch_bounds__(kDeWavesMax * kWave)
 __attribute__((amdgpu_waves_per_eu(de_min_occupancy<MODEL, W, VARIANT>(), 8))) void de_semblance_kernel(DeArgs a) {
@@ -328,35 +363,145 @@ __attribute__((amdgpu_waves_per_eu(de_min_occupancy<MODEL, W, VARIANT>(), 8))) v
             atomicAdd(a.not_used + g, (unsigned long long)rejected);
     }
     if (a.gen_end < a.G || wave != 0 || !active) return;
-    const int cur = (a.G - 1) & 1;
-    // selectBestIndividuals*: first strict maximum of S over the population
-    float best = -1.0f, bstack = 0.0f;
-    int bi = -1;
-    for (int i = 0; i < NP; ++i) {
-        const float S = *rec(cur, i, D);
-        if (S > best) {
-            best = S;
-            bstack = *rec(cur, i, D + 1);
-            bi = i;
+    de_report<D>(a, g, s, rec);
+}
+
+// The same run spread over more of the chip: a workgroup takes T = 16 consecutive t0 samples,
+// and a wave's lanes split into four groups with an individual each, so that (with up to
+// twelve waves) the whole population of a sample is evaluated at once, one individual per
+// lane.  Workspace rows, random streams, donors and selections are those of
+// de_semblance_kernel, so the results are the same bits, and a run may change kernels between
+// generation ranges.
+//
+// One midpoint has ns/64 workgroups in de_semblance_kernel and each wave evaluates its
+// individuals one pair after the other: 1001 samples, NP = 32, took 54.4 ms on 16 CUs
+// (ZO-CRS, FP32, G = 50) where this kernel takes 15.1.  For CMP and OCT it is the faster one
+// at every size (OCT, NP = 48, 24 midpoints 88.0 -> 68.4 ms, NP = 32, 128 midpoints 58.5 ->
+// 44.6 ms; CMP, 60 midpoints 6.2 -> 5.1 ms): one candidate's registers and windows per lane,
+// neighbouring lanes on neighbouring samples of one individual, short workgroups.  Two
+// individuals per lane share ZO-CRS's long trace loop better once the chip is full (128
+// midpoints: 62.3 against 67.5 ms here; 32 midpoints, 512 workgroups: 90.5 against 88.4), so
+// it keeps de_semblance_kernel above 512 workgroups of it.  (OCT at T = 8/16/32: 77.8/68.4/
+// 72.6 ms; at eight waves, two passes over 48 individuals, 84.7; at five waves per SIMD 88.8.)
+constexpr int kDeSpreadTl = 4;
+constexpr int kDeSpreadWaves = 12;
+constexpr long long kDeSpreadZocrsTiles = 512;
+template <int MODEL>
+constexpr bool de_spread_always() { return MODEL != HSS_ZOCRS; }
+
+template <int MODEL, int W, int VARIANT, int STORAGE>
+__global__ __launch_bounds__(kDeSpreadWaves * kWave)
+__attribute__((amdgpu_waves_per_eu(6, 8))) void de_spread_kernel(DeArgs a) {
+    constexpr int D = MODEL == HSS_CMP ? 1 : (MODEL == HSS_ZOCRS ? 3 : 2);
+    constexpr int REC = D + 2;  // D parameters, S, stack
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    constexpr int T = 1 << kDeSpreadTl;
+    const int wg_per_mid = (a.e.ns + T - 1) / T;
+    const int blk = logical_block(blockIdx.x, gridDim.x);
+    const int slot = blk / wg_per_mid;
+    const int g = launch_midpoint(a.morder, a.nmid, slot);
+    if (g < 0) return;  // (the whole workgroup)
+    const int s0 = (blk - slot * wg_per_mid) * T;
+    const int s = s0 + (lane & (T - 1));
+    const int ns = a.e.ns;
+    const bool active = s < ns;
+    const float t0 = (float)s * a.e.dt;
+    const EvalCtx e = midpoint_ctx(a.e, a.mbeg, a.mcnt, a.mm0, g);
+    const uint32_t stream = a.stream_base + (uint32_t)g;
+    const int NP = a.NP;
+    constexpr int per_wave = kWave / T;
+    const int per_pass = per_wave * ((int)blockDim.x / kWave);
+    const int first = wave * per_wave + lane / T;  // the lane's individual of a pass
+    // the workspace column of sample s in de_semblance_kernel's 64-sample tiles
+    float *const column = a.ws +
+                          ((size_t)g * a.ntiles + s0 / kWave) * 2 * NP * REC * kWave + s % kWave;
+    auto rec = [&](int buf, int i, int f) -> float * {
+        return column + ((size_t)(buf * NP + i) * REC + f) * kWave;
+    };
+    __shared__ std::conditional_t<de_compact<MODEL, VARIANT>(), OctRuns, int> runs;
+    bool by_runs = false;
+    if constexpr (de_compact<MODEL, VARIANT>())
+        by_runs = load_oct_runs(e, STORAGE == HSS_F32 ? 4 : 2, runs);
+    uint64_t rejected = 0;  // the wave's rejections (uniform)
+    auto eval = [&](const Candidate &k, bool on, float *S, float *stk) {
+        const Candidate kc[1] = {k};
+        const bool on1[1] = {on};
+        float S1[1], T1[1];
+        unsigned rej = 0;  // on the wave's lowest active lane
+        const bool live = active && on;
+        if constexpr (de_compact<MODEL, VARIANT>()) {
+            if (by_runs)
+                evaluate_oct_runs<W, VARIANT, STORAGE, false, 1>(e, runs, t0, kc, on1, 0.0f, live,
+                                                                 S1, T1, &rej);
+            else
+                evaluate_n<MODEL, W, VARIANT, STORAGE, false, 1, kDeSegments, kDeOctKeep>(
+                    e, t0, t0 * t0, kc, on1, 0.0f, live, nullptr, S1, T1, &rej);
+        } else if (STORAGE == HSS_BF16 && e.scale == nullptr)
+            evaluate_n<MODEL, W, VARIANT, STORAGE, false, 1, kDeSegments, kDeOctKeep, false>(
+                e, t0, t0 * t0, kc, on1, 0.0f, live, nullptr, S1, T1, &rej);
+        else
+            evaluate_n<MODEL, W, VARIANT, STORAGE, false, 1, kDeSegments, kDeOctKeep>(
+                e, t0, t0 * t0, kc, on1, 0.0f, live, nullptr, S1, T1, &rej);
+        if constexpr (MODEL == HSS_OCT) {
+            for (uint64_t m = __builtin_amdgcn_ballot_w64(rej != 0u); m; m &= m - 1)
+                rejected += (uint32_t)__builtin_amdgcn_readlane((int)rej, __builtin_ctzll(m));
         }
-    }
-    float *res = a.result + (size_t)g * (2 + D) * ns;
-    res[s] = best;
-    res[ns + s] = bi >= 0 ? bstack : 0.0f;
+        *S = S1[0];
+        *stk = T1[0];
+    };
+    for (int gen = a.gen_begin; gen < a.gen_end; ++gen) {
+        const int cur = (gen - 1) & 1, next = gen & 1;
+        for (int p0 = 0; p0 < NP; p0 += per_pass) {
+            // (a lane past the population works on the last individual and keeps nothing; so
+            // does one past the trace, whose column lies in the last tile's padding)
+            const bool on = p0 + first < NP;
+            const int i = min(p0 + first, NP - 1);
+            float x[D];
+            if (gen == 0) {
+                float u[4];
+                de_uniforms<D>(a, (uint32_t)s, stream, i, 0, u);
 #pragma unroll
-    for (int d = 0; d < D; ++d) res[(2 + d) * ns + s] = bi >= 0 ? *rec(cur, bi, d) : 0.0f;
-    if (a.pop_x) {
-        for (int i = 0; i < NP; ++i)
+                for (int d = 0; d < D; ++d) x[d] = a.lo[d] + u[d] * (a.hi[d] - a.lo[d]);
+            } else {
+                constexpr int NQ = 4 * D + 1;
+                float u[NQ];
+                de_uniforms<NQ>(a, (uint32_t)s, stream, i, gen, u);
+                const float np1 = (float)(NP - 1);
+                const unsigned l = (unsigned)(u[3 * D] * (float)(D - 1));
 #pragma unroll
-            for (int d = 0; d < D; ++d)
-                a.pop_x[(((size_t)g * ns + s) * NP + i) * D + d] = *rec(cur, i, d);
-    }
-    if (a.pop_fx) {
-        for (int i = 0; i < NP; ++i) {
-            a.pop_fx[(((size_t)g * ns + s) * NP + i) * 2] = *rec(cur, i, D);
-            a.pop_fx[(((size_t)g * ns + s) * NP + i) * 2 + 1] = *rec(cur, i, D + 1);
+                for (int d = 0; d < D; ++d) {
+                    const unsigned r1 = (unsigned)(u[3 * d] * np1);
+                    const unsigned r2 = (unsigned)(u[3 * d + 1] * np1);
+                    const unsigned r3 = (unsigned)(u[3 * d + 2] * np1);
+                    float nv = *rec(cur, r1, d) + kDeF * (*rec(cur, r2, d) - *rec(cur, r3, d));
+                    nv = fminf(nv, a.hi[d]);
+                    nv = fmaxf(nv, a.lo[d]);
+                    const float r = u[3 * D + 1 + d];
+                    x[d] = (r > kDeCR && l != (unsigned)d) ? *rec(cur, i, d) : nv;
+                }
+            }
+            float S, stk;
+            eval(de_candidate<MODEL>(x), on, &S, &stk);
+            if (!on || !active) continue;
+            if (gen > 0 && !(S > *rec(cur, i, D))) {
+#pragma unroll
+                for (int f = 0; f < REC; ++f) *rec(next, i, f) = *rec(cur, i, f);
+            } else {
+#pragma unroll
+                for (int d = 0; d < D; ++d) *rec(next, i, d) = x[d];
+                *rec(next, i, D) = S;
+                *rec(next, i, D + 1) = stk;
+            }
         }
+        __syncthreads();
     }
+    if (MODEL == HSS_OCT && a.not_used) {
+        if (lane == 0 && rejected) atomicAdd(a.not_used + g, (unsigned long long)rejected);
+    }
+    // the lanes of the first group report their samples
+    if (a.gen_end < a.G || first != 0 || !active) return;
+    de_report<D>(a, g, s, rec);
 }
 
 template <int MODEL>
@@ -364,9 +509,26 @@ int launch_de(const DeArgs &a, int n_mid, int variant, int storage, hipStream_t 
     int st = HSS_OK;
     const unsigned blocks = (unsigned)n_mid * (unsigned)a.ntiles;
     if (blocks == 0) return HSS_OK;
+    constexpr int T = 1 << kDeSpreadTl, per_wave = kWave / T;
+    const long long spread = (long long)n_mid * ((a.e.ns + T - 1) / T);
+    const bool spread_it = (de_spread_always<MODEL>() || (long long)blocks <= kDeSpreadZocrsTiles) &&
+                           spread <= 0x7fffffffll;
+    // the waves that take the population in the fewest equal passes
+    const int need = (a.NP + per_wave - 1) / per_wave;
+    const int passes = (need + kDeSpreadWaves - 1) / kDeSpreadWaves;
+    const int waves = (need + passes - 1) / passes;
     int rc = dispatch_storage(storage, [&](auto S) {
         st = dispatch_variant(variant, [&](auto V) {
             dispatch_window(a.e.w, fast_index_verified(a.e.dt, a.e.tau, stream), [&](auto Wc) {
+                if constexpr (decltype(Wc)::value > 0 && decltype(V)::value != HSS_KAHAN) {
+                    if (spread_it) {
+                        hipLaunchKernelGGL((de_spread_kernel<MODEL, decltype(Wc)::value,
+                                                             decltype(V)::value, decltype(S)::value>),
+                                           dim3((unsigned)spread), dim3(waves * kWave), 0, stream,
+                                           a);
+                        return;
+                    }
+                }
                 hipLaunchKernelGGL((de_semblance_kernel<MODEL, decltype(Wc)::value,
                                                         decltype(V)::value, decltype(S)::value>),
                                    dim3(blocks), dim3(de_waves<MODEL>() * kWave), 0, stream, a);
