@@ -311,12 +311,11 @@ int hss_stretch_free(const hss_traces *traces, const hss_midpoints *mids, int mo
     a.vparams = d_vparams;
     for (int q = 0; q < nN; ++q) a.nvals[q] = nvals[q];
     a.nN = nN;
-    a.ntiles = tiles_of(traces->ns);
     a.result = d_result;
     a.sembl = d_sembl;
     a.stack = d_stack;
     a.not_used = d_not_used;
-    if ((unsigned long long)mids->n * (unsigned long long)a.ntiles > 0x7fffffffULL)
+    if ((unsigned long long)mids->n * (unsigned long long)tiles_of(traces->ns) > 0x7fffffffULL)
         return HSS_ERR_INVALID_SIZE;
     hipStream_t st = (hipStream_t)stream;
     switch (model) {
