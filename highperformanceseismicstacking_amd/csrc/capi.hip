@@ -206,7 +206,7 @@ int hss_grid_semblance(const hss_traces *traces, const hss_midpoints *mids, int 
     };
     if (!grid_shape_pinned(model, traces->w, variant, traces->storage) &&
         spread_wanted(model, traces->storage, (long long)mids->n * a.ntiles)) {
-        const int tl = spread_tl(model, mids->n, traces->ns, P);
+        const int tl = spread_tl(model, mids->n, traces->ns, traces->w, P);
         int status = HSS_OK;
         bool done;
         switch (model) {

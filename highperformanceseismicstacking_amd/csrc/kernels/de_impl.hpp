@@ -517,26 +517,33 @@ int launch_de(const DeArgs &a, int n_mid, int variant, int storage, hipStream_t 
     const int need = (a.NP + per_wave - 1) / per_wave;
     const int passes = (need + kDeSpreadWaves - 1) / kDeSpreadWaves;
     const int waves = (need + passes - 1) / passes;
+    int st_launch = HSS_OK;
     int rc = dispatch_storage(storage, [&](auto S) {
         st = dispatch_variant(variant, [&](auto V) {
             dispatch_window(a.e.w, fast_index_verified(a.e.dt, a.e.tau, stream), [&](auto Wc) {
-                if constexpr (decltype(Wc)::value > 0 && decltype(V)::value != HSS_KAHAN) {
+                constexpr int VV = decltype(V)::value, SS = decltype(S)::value,
+                              WW = window_of<decltype(Wc)::value, VV, true>();
+                if constexpr (WW > 0 && VV != HSS_KAHAN) {
                     if (spread_it) {
-                        hipLaunchKernelGGL((de_spread_kernel<MODEL, decltype(Wc)::value,
-                                                             decltype(V)::value, decltype(S)::value>),
+                        hipLaunchKernelGGL((de_spread_kernel<MODEL, WW, VV, SS>),
                                            dim3((unsigned)spread), dim3(waves * kWave), 0, stream,
                                            a);
                         return;
                     }
                 }
-                hipLaunchKernelGGL((de_semblance_kernel<MODEL, decltype(Wc)::value,
-                                                        decltype(V)::value, decltype(S)::value>),
-                                   dim3(blocks), dim3(de_waves<MODEL>() * kWave), 0, stream, a);
+                // (CMP and OCT are spread: what is left is compensated or has no compiled
+                // window)
+                if constexpr (!(de_spread_always<MODEL>() && WW > 0 && VV != HSS_KAHAN))
+                    hipLaunchKernelGGL((de_semblance_kernel<MODEL, WW, VV, SS>), dim3(blocks),
+                                       dim3(de_waves<MODEL>() * kWave), 0, stream, a);
+                else
+                    st_launch = HSS_ERR_INVALID_SIZE;  // 2^31 workgroups: no workspace holds them
             });
         });
     });
     if (rc != HSS_OK) return rc;
     if (st != HSS_OK) return st;
+    if (st_launch != HSS_OK) return st_launch;
     return hip_status(hipGetLastError());
 }
 

@@ -12,14 +12,17 @@ int launch_grid_cmp_staged(const GridArgs &a, int n_slots, int variant, int stor
     int rc = dispatch_storage(storage, [&](auto S) {
         st = dispatch_variant(variant, [&](auto V) {
             dispatch_window(a.e.w, fast_index_verified(a.e.dt, a.e.tau, stream), [&](auto Wc) {
-                constexpr int WW = decltype(Wc)::value, VV = decltype(V)::value,
-                              SS = decltype(S)::value;
-                if (cpl == 2 && WW > 0)
-                    hipLaunchKernelGGL((grid_staged_kernel<WW, VV, SS, 2>), dim3(blocks),
-                                       dim3(kStagedThreads), 0, stream, a);
-                else
-                    hipLaunchKernelGGL((grid_staged_kernel<WW, VV, SS, 1>), dim3(blocks),
-                                       dim3(kStagedThreads), 0, stream, a);
+                constexpr int VV = decltype(V)::value, SS = decltype(S)::value,
+                              WW = window_of<decltype(Wc)::value, VV, true>();
+                if constexpr (WW > 0 && !wide_window(WW)) {
+                    if (cpl == 2) {
+                        hipLaunchKernelGGL((grid_staged_kernel<WW, VV, SS, 2>), dim3(blocks),
+                                           dim3(kStagedThreads), 0, stream, a);
+                        return;
+                    }
+                }
+                hipLaunchKernelGGL((grid_staged_kernel<WW, VV, SS, 1>), dim3(blocks),
+                                   dim3(kStagedThreads), 0, stream, a);
             });
         });
     });

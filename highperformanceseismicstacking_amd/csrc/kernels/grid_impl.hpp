@@ -211,8 +211,8 @@ int launch_grid(const GridArgs &a, int n_slots, int variant, int storage, int cp
     int rc = dispatch_storage(storage, [&](auto S) {
         st = dispatch_variant(variant, [&](auto V) {
             dispatch_window(a.e.w, fast_index_verified(a.e.dt, a.e.tau, stream), [&](auto Wc) {
-                constexpr int WW = decltype(Wc)::value, VV = decltype(V)::value,
-                              SS = decltype(S)::value;
+                constexpr int VV = decltype(V)::value, SS = decltype(S)::value,
+                              WW = window_of<decltype(Wc)::value, VV, false>();
                 if (cpl == 2 && WW > 0)
                     hipLaunchKernelGGL((grid_semblance_kernel<MODEL, WW, VV, SS, 2>), dim3(blocks),
                                        dim3(kGridThreads), 0, stream, a);

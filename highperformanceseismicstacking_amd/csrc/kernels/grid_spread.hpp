@@ -23,7 +23,8 @@ namespace hss {
 
 constexpr int kSpreadWaves = 8;
 constexpr int kSpreadThreads = kSpreadWaves * kWave;
-constexpr int kSpreadCpl = 2;
+// Candidates per lane.
+constexpr int spread_cpl(int w) { return w > 15 ? 1 : 2; }
 // Register budget, as waves per SIMD (a workgroup is two of them).  Windows of up to 11 samples
 // of CMP and ZO-CRS fit six (39.9 against 42.8 ms at four, ZO-CRS, 24 midpoints); OCT, whose
 // terms would spill, and wider windows take four (OCT 76 ms, 79 at six; w = 15: 43 against 59
@@ -35,7 +36,7 @@ template <int MODEL, int W, int VARIANT, int STORAGE>
 __global__ __launch_bounds__(kSpreadThreads)
 __attribute__((amdgpu_waves_per_eu(spread_min_waves<MODEL, W>(), 8))) void grid_spread_kernel(GridArgs a) {
     constexpr int NP = MODEL == HSS_CMP ? 1 : (MODEL == HSS_ZOCRS ? 3 : 2);
-    constexpr int CPL = kSpreadCpl;
+    constexpr int CPL = spread_cpl(W);
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
     const int T = 1 << a.tl;  // t0 samples per workgroup
@@ -128,16 +129,16 @@ __attribute__((amdgpu_waves_per_eu(spread_min_waves<MODEL, W>(), 8))) void grid_
 }
 
 // log2 of T.  The workgroups should outnumber the CUs eight times, for a launch that ends
-// evenly; below that T halves down to 4.  T also stays at 1024/P or above, where one round
-// takes all P candidates (64 candidates on 12 midpoints: T = 16 190 us, T = 8, half of the
+// evenly; below that T halves down to 4.  T also stays at 512*CPL/P or above, where one
+// round takes all P candidates (64 candidates on 12 midpoints: T = 16 190 us, T = 8, half of the
 // lanes idle, 270 us).  T = 16 is the largest that pays (ZO-CRS, 100 midpoints: 51/45/41.9/
 // 41.4 ms at 64/32/16/8), 32 for OCT (100 midpoints: 62/57.6/59.1/75 ms), whose runs visit
 // the traces that any of a wave's candidates keeps.
 constexpr int kSpreadWorkgroups = 2048;
-inline int spread_tl(int model, int n_slots, int ns, int P) {
+inline int spread_tl(int model, int n_slots, int ns, int w, int P) {
     int tl = model == HSS_OCT ? 5 : 4;
     while (tl > 2 && (long long)n_slots * ((ns + (1 << tl) - 1) >> tl) < kSpreadWorkgroups) --tl;
-    while (tl < 6 && (2048ll >> tl) > P) ++tl;
+    while (tl < 6 && ((long long)(2 * kSpreadThreads * spread_cpl(w)) >> tl) > P) ++tl;
     return tl;
 }
 

@@ -63,8 +63,13 @@ int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, in
                      hipStream_t stream, const std::function<int(GridShape, int)> &launch,
                      GridShape *shape_out);
 
-// Calls f(std::integral_constant<int, W>) for the compiled window sizes; any other w
-// (odd, <= 32), or fast = false, goes to the runtime-w instantiation W = 0.
+// Calls f(std::integral_constant<int, W>) for the compiled window sizes, every odd one from 3
+// to 31; w = 1, or fast = false, goes to the runtime-w instantiation W = 0.  Only 5 to 15 are
+// compiled for every kernel and variant; the others (wide_window) for the contracted and exact
+// sums of the kernels that a launch takes by itself, with one candidate per lane.  (w = 21 by
+// the runtime-w kernels against compiled ones: CMP grid, 60 midpoints, 256 candidates 8.1 ->
+// 3.7 ms; ZO-CRS differential evolution, 8 midpoints 82 -> 11.2 ms; OCT grid, 20 midpoints
+// 120 -> 12.8 ms, both with their spread kernels, which need a compiled window.)
 template <class F>
 inline void dispatch_window(int w, bool fast, F &&f) {
     if (!fast) {
@@ -72,14 +77,22 @@ inline void dispatch_window(int w, bool fast, F &&f) {
         return;
     }
     switch (w) {
-        case 5: f(std::integral_constant<int, 5>{}); break;
-        case 7: f(std::integral_constant<int, 7>{}); break;
-        case 9: f(std::integral_constant<int, 9>{}); break;
-        case 11: f(std::integral_constant<int, 11>{}); break;
-        case 13: f(std::integral_constant<int, 13>{}); break;
-        case 15: f(std::integral_constant<int, 15>{}); break;
+#define HSS_WINDOW(W) \
+    case W: f(std::integral_constant<int, W>{}); break;
+        HSS_WINDOW(3) HSS_WINDOW(5) HSS_WINDOW(7) HSS_WINDOW(9) HSS_WINDOW(11)
+        HSS_WINDOW(13) HSS_WINDOW(15) HSS_WINDOW(17) HSS_WINDOW(19) HSS_WINDOW(21)
+        HSS_WINDOW(23) HSS_WINDOW(25) HSS_WINDOW(27) HSS_WINDOW(29) HSS_WINDOW(31)
+#undef HSS_WINDOW
         default: f(std::integral_constant<int, 0>{}); break;
     }
+}
+
+constexpr bool wide_window(int W) { return W == 3 || W > 15; }
+
+// The window size a kernel is instantiated for: W, or 0 where only 5 to 15 are compiled.
+template <int W, int VARIANT, bool WIDE>
+constexpr int window_of() {
+    return wide_window(W) && (!WIDE || VARIANT == HSS_KAHAN) ? 0 : W;
 }
 
 template <class F>

@@ -241,8 +241,10 @@ int launch_sf(const SfArgs &args, int n_mid, int variant, int storage, hipStream
             // (dt: see sqrt_time)
             const bool fast = a.e.dt >= 0x1.0p-20f && fast_index_verified(a.e.dt, a.e.tau, stream);
             dispatch_window(a.e.w, fast, [&](auto Wc) {
-                hipLaunchKernelGGL((sf_semblance_kernel<MODEL, decltype(Wc)::value,
-                                                        decltype(V)::value, decltype(S)::value>),
+                constexpr int VV = decltype(V)::value;
+                hipLaunchKernelGGL((sf_semblance_kernel<MODEL,
+                                                        window_of<decltype(Wc)::value, VV, true>(),
+                                                        VV, decltype(S)::value>),
                                    dim3((unsigned)blocks), dim3(threads), lds, stream, a);
             });
         });

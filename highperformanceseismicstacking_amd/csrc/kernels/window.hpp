@@ -382,7 +382,10 @@ struct Window {
     __device__ __forceinline__ void add16(const uint32_t *roww, unsigned rpar, unsigned k,
                                           float f, float sc, int slot = 0) {
         static_assert(W > 0, "add16 needs a compiled window size");
-        if constexpr (VARIANT != HSS_EXACT && STORAGE == HSS_F16 && FACTORED) {
+        // windows of other sizes than 5 to 15 samples keep the form of the runtime-w kernel
+        // they came from, whose samples are scaled one by one
+        constexpr bool FACTOR = FACTORED && W >= 5 && W <= 15;
+        if constexpr (VARIANT != HSS_EXACT && STORAGE == HSS_F16 && FACTOR) {
             // as below, with y1 - y0 formed as fma(y1, one, -y0) = RN(y1 - y0): the same
             // bits, but an FMA reads both halves straight from the words (v_fma_mix_f32),
             // where a subtraction needs both converted first.  `one` is 1.0 hidden from the
@@ -405,7 +408,11 @@ struct Window {
         float y[W + 1];
         read16<STORAGE, W>(roww, rpar, k, y);
         if constexpr (VARIANT != HSS_EXACT) {
-            if constexpr (!FACTORED) {
+            if constexpr (!FACTOR) {
+                if constexpr (FACTORED) {
+#pragma unroll
+                    for (int j = 0; j <= W; ++j) y[j] = y[j] * sc;
+                }
                 sum(y, f, slot);
                 used++;
                 return;
