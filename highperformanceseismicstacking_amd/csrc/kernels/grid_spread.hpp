@@ -10,8 +10,8 @@
 // one lane group are neighbours, so windows stay close together where T is small.  Measured
 // (T in brackets; before -> here): one 60-trace gather, 256 candidates [4] 425 -> 51 us (the
 // staged kernel); ZO-CRS, 24 midpoints, BF16 [16] 119 -> 39.9 ms, 200 midpoints 97 -> 82 ms;
-// OCT, 30 midpoints, FP16 [16] 188 -> 76 ms, 250 midpoints [32] 204 -> 137 ms; OCT, 30
-// midpoints in the reference's order, EXACT 105 -> 74 ms.  What bounds it then is VALU issue:
+// OCT, 30 midpoints, FP16 [4] 188 -> 48 ms (76 without the slopes' order below), 250 midpoints
+// 204 -> 101 ms; OCT, 30 midpoints in the reference's order, EXACT 105 -> 60 ms.  What bounds it then is VALU issue:
 // the 16-bit lanes widen and scale every sample of their own windows, the price of not sharing
 // LDS segments.
 #pragma once
@@ -31,6 +31,23 @@ constexpr int spread_cpl(int w) { return w > 15 ? 1 : 2; }
 // at two, which leaves one workgroup per CU).
 template <int MODEL, int W>
 constexpr int spread_min_waves() { return MODEL == HSS_OCT || W > 11 ? 4 : 6; }
+
+// OCT candidates {c, slope}: the smallest d > 0, up to 256, whose slope is candidate 0's (its
+// bit pattern), if it divides P; else 1.  Every lane of the wave calls it.
+__device__ __forceinline__ int slope_period(const float *__restrict__ params, int P) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t first = __float_as_uint(params[1]);
+    for (int d0 = 1; d0 < P && d0 <= 256; d0 += kWave) {
+        const int d = d0 + lane;
+        const unsigned long long same = __builtin_amdgcn_ballot_w64(
+            d < P && __float_as_uint(params[2 * min(d, P - 1) + 1]) == first);
+        if (same) {
+            const int period = d0 + __builtin_ctzll(same);
+            return P % period == 0 ? period : 1;
+        }
+    }
+    return 1;
+}
 
 template <int MODEL, int W, int VARIANT, int STORAGE>
 __global__ __launch_bounds__(kSpreadThreads)
@@ -58,14 +75,27 @@ __attribute__((amdgpu_waves_per_eu(spread_min_waves<MODEL, W>(), 8))) void grid_
     unsigned long long rejected = 0;
     bool by_runs = false;
     if constexpr (MODEL == HSS_OCT) by_runs = oct_offset_runs_long(e);
+    // The candidates in the order the lanes take them: rank -> candidate, a permutation.
+    // OCT: where the first slope comes again after `period` candidates (a grid, slope
+    // fastest), all candidates of a slope one after the other, so that a wave's candidates
+    // displace midpoints alike and its runs visit few traces.
+    const int period = MODEL == HSS_OCT ? slope_period(a.params, a.P) : 1;
+    const int per_slope = a.P / period;
+    auto candidate_of = [&](int rank) {
+        if constexpr (MODEL != HSS_OCT) return rank;
+        const int sl = rank / per_slope;
+        return (rank - sl * per_slope) * period + sl;
+    };
     for (int r0 = 0; r0 < a.P; r0 += groups * CPL) {
         const int q0 = r0 + grp * CPL;
         Candidate k[CPL];
         bool on[CPL];
+        int cand[CPL];
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             on[c] = q0 + c < a.P;
-            k[c] = load_candidate<MODEL>(a.params, min(q0 + c, a.P - 1));
+            cand[c] = candidate_of(min(q0 + c, a.P - 1));
+            k[c] = load_candidate<MODEL>(a.params, cand[c]);
         }
         float S[CPL], stk[CPL];
         unsigned rej = 0;
@@ -76,10 +106,11 @@ __attribute__((amdgpu_waves_per_eu(spread_min_waves<MODEL, W>(), 8))) void grid_
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             if (!on[c]) continue;
-            const int q = q0 + c;
+            const int q = cand[c];
             if (a.sembl) a.sembl[((size_t)g * ns + s) * a.P + q] = S[c];
             if (a.stack) a.stack[((size_t)g * ns + s) * a.P + q] = stk[c];
-            if (S[c] > best) {
+            // the first strict maximum, in whatever order the candidates come
+            if (S[c] > best || (MODEL == HSS_OCT && S[c] == best && q < bidx)) {
                 best = S[c];
                 bstack = stk[c];
                 bidx = q;
@@ -132,11 +163,11 @@ __attribute__((amdgpu_waves_per_eu(spread_min_waves<MODEL, W>(), 8))) void grid_
 // evenly; below that T halves down to 4.  T also stays at 512*CPL/P or above, where one
 // round takes all P candidates (64 candidates on 12 midpoints: T = 16 190 us, T = 8, half of the
 // lanes idle, 270 us).  T = 16 is the largest that pays (ZO-CRS, 100 midpoints: 51/45/41.9/
-// 41.4 ms at 64/32/16/8), 32 for OCT (100 midpoints: 62/57.6/59.1/75 ms), whose runs visit
-// the traces that any of a wave's candidates keeps.
+// 41.4 ms at 64/32/16/8), 4 for OCT (30 midpoints, 1024 candidates: 56/50.4/48.2 ms at 16/8/4),
+// where a wave of few samples and many candidates of one slope keeps few traces of a run.
 constexpr int kSpreadWorkgroups = 2048;
 inline int spread_tl(int model, int n_slots, int ns, int w, int P) {
-    int tl = model == HSS_OCT ? 5 : 4;
+    int tl = model == HSS_OCT ? 2 : 4;
     while (tl > 2 && (long long)n_slots * ((ns + (1 << tl) - 1) >> tl) < kSpreadWorkgroups) --tl;
     while (tl < 6 && ((long long)(2 * kSpreadThreads * spread_cpl(w)) >> tl) > P) ++tl;
     return tl;

@@ -44,7 +44,7 @@ def _case(form, n, ns):
 @pytest.mark.parametrize("n,ns,counts,tau", [(1, 50, (3, 1, 1), 2), (2, 130, (5, 3, 2), 5),
                                              (1, 333, (150, 2, 1), 7), (9, 403, (17, 2, 2), 3),
                                              (2, 150, (5, 3, 2), 1), (2, 150, (7, 3, 2), 10),
-                                             (1, 140, (70, 1, 1), 15)])
+                                             (1, 140, (70, 1, 1), 15), (1, 90, (12, 7, 2), 4)])
 def test_spread_equals_one_tile(form, storage, variant, n, ns, counts, tau):
     import torch
     line, model, b, c, m0, index, h0, apm = _case(form, n, ns)
