@@ -297,7 +297,9 @@ struct GradSums {
 // S, stack and dS/dtheta for one lane's own parameter point.  FMA arithmetic (as
 // HSS_FAST); per-lane windows are read with per-lane loads.  Every lane of the wave must
 // call it (the trace geometry is broadcast across the wave).
-template <int MODEL, int W, int STORAGE>
+// BATCH: traces whose windows are requested before the first is summed (kAdjBatch; traces must
+// then be longer than the window, and the model CMP or ZO-CRS).
+template <int MODEL, int W, int STORAGE, int BATCH = 1>
 __device__ __forceinline__ void evaluate_grad(const EvalCtx &e, float t0, float t0sq,
                                               const Candidate &k, bool active, float *S,
                                               float *stack, float *grad) {
@@ -327,6 +329,53 @@ __device__ __forceinline__ void evaluate_grad(const EvalCtx &e, float t0, float 
                                    : TraceGeom{0.0f, 0.0f, 0.0f};
         const float sc_l = (scaled && have) ? e.scale[ti_l] : 1.0f;
         const int nchunk = min(kWave, e.cnt - j0);
+        if constexpr (BATCH > 1) {
+            static_assert(W > 0 && MODEL != HSS_OCT, "compiled windows of CMP and ZO-CRS");
+            for (int jb = 0; jb < nchunk; jb += BATCH) {
+                float f[BATCH], gi[BATCH][D], y[BATCH][N + 1], sc[BATCH];
+                bool use[BATCH];
+#pragma unroll
+                for (int b = 0; b < BATCH; ++b) {
+                    const int jj = min(jb + b, nchunk - 1);
+                    const size_t trace0 =
+                        (size_t)__builtin_amdgcn_readlane(ti_l, jj) * (size_t)e.ns;
+                    const TraceGeom tg{bcast(g_l.m, jj), bcast(g_l.h, jj), bcast(g_l.h2, jj)};
+                    sc[b] = scaled ? bcast(sc_l, jj) : 1.0f;
+                    float t = 0.0f, dtd[D];
+                    const bool ok = traveltime_grad<MODEL, FASTIDX>(tg, t0, t0sq, e.m0, e.h0, e.apm,
+                                                                    k, &t, dtd, false, kept);
+                    int first;
+                    const bool in =
+                        window_index<FASTIDX>(t, e.dt, e.inv_dt, e.ib, e.tau, &first, &f[b]);
+                    use[b] = ok & in & active & (jb + b < nchunk);
+#pragma unroll
+                    for (int m = 0; m < D; ++m) gi[b][m] = dtd[m] * e.inv_dt;
+                    // a lane without a window there reads the trace's first one
+                    const uint32_t at = use[b] ? (uint32_t)first : 0u;
+                    if constexpr (STORAGE == HSS_F32) {
+                        const float *p = (const float *)at_bytes((const float *)e.samples + trace0,
+                                                                 4u * at);
+#pragma unroll
+                        for (int j = 0; j <= N; ++j) y[b][j] = p[j];
+                    } else {
+                        const unsigned rpar = (unsigned)trace0 & 1u;
+                        read16<STORAGE, W>(
+                            (const uint32_t *)((const uint16_t *)e.samples + (trace0 - rpar)),
+                            rpar, at, y[b]);
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < BATCH; ++b) {
+                    if (!use[b]) continue;
+                    if constexpr (STORAGE != HSS_F32) {
+#pragma unroll
+                        for (int j = 0; j <= N; ++j) y[b][j] = y[b][j] * sc[b];
+                    }
+                    sums.add(y[b], f[b], gi[b], e.w);
+                }
+            }
+            continue;
+        }
         for (int jj = 0; jj < nchunk; ++jj) {
             const int ti = __builtin_amdgcn_readlane(ti_l, jj);
             TraceGeom tg;
@@ -472,7 +521,7 @@ template <int MODEL>
 constexpr int adj_waves() { return MODEL == HSS_OCT ? 4 : 1; }
 
 // Where a wave of an adjoint kernel works, and its evaluation of the gradient there.
-template <int MODEL, int W, int STORAGE>
+template <int MODEL, int W, int STORAGE, int BATCH>
 struct AdjointWave {
     EvalCtx e;
     int g, s, ns;
@@ -509,7 +558,7 @@ struct AdjointWave {
                 return;
             }
         }
-        evaluate_grad<MODEL, W, STORAGE>(e, t0, t0 * t0, k, active, S, stack, grad);
+        evaluate_grad<MODEL, W, STORAGE, BATCH>(e, t0, t0 * t0, k, active, S, stack, grad);
     }
 };
 
@@ -528,10 +577,10 @@ __device__ __forceinline__ void grad_to_v(const float *p, float *g) {
     g[0] = g[0] * (-8.0f / (p[0] * p[0] * p[0]));
 }
 
-template <int MODEL, int W, int STORAGE>
+template <int MODEL, int W, int STORAGE, int BATCH>
 __global__ __launch_bounds__(adj_waves<MODEL>() * kWave) void gradient_kernel(AdjointArgs a) {
     constexpr int D = model_np<MODEL>();
-    AdjointWave<MODEL, W, STORAGE> wv;
+    AdjointWave<MODEL, W, STORAGE, BATCH> wv;
     if (!wv.init(a)) return;
     const int g = wv.g, s = wv.s, ns = wv.ns;
     const EvalCtx &e = wv.e;
@@ -561,10 +610,10 @@ __global__ __launch_bounds__(adj_waves<MODEL>() * kWave) void gradient_kernel(Ad
 //   dx = r * dS/dx / (|dS/dx|^2 + mu),
 // kept when S increases (mu /= 3), rejected otherwise (mu *= 4); mu starts at |dS/dx|^2.
 // S never decreases; the point stays in the box.
-template <int MODEL, int W, int STORAGE>
+template <int MODEL, int W, int STORAGE, int BATCH>
 __global__ __launch_bounds__(adj_waves<MODEL>() * kWave) void polish_kernel(AdjointArgs a) {
     constexpr int D = model_np<MODEL>();
-    AdjointWave<MODEL, W, STORAGE> wv;
+    AdjointWave<MODEL, W, STORAGE, BATCH> wv;
     if (!wv.init(a)) return;
     const int g = wv.g, s = wv.s, ns = wv.ns;
     const EvalCtx &e = wv.e;
@@ -622,6 +671,16 @@ __global__ __launch_bounds__(adj_waves<MODEL>() * kWave) void polish_kernel(Adjo
     for (int m = 0; m < D; ++m) out[(2 + m) * ns + s] = p[m];
 }
 
+// Launches of at most two waves per SIMD wait on one trace's window loads at a time: four traces'
+// windows (two for the compiled windows above 15 samples, whose rows are the registers) are then
+// requested together and summed in the lists' order, so the results keep their bits. Six polish
+// steps, one trace at a time | batched: CMP, 5 samples, F32, 2 x 24 waves 0.246 | 0.181 ms,
+// 80 x 24 0.310 | 0.222; ZO-CRS, 5 samples, bf16, 30 x 16 waves 3.48 | 2.91, 100 x 16 4.74 | 3.98;
+// 21 samples, F32, 30 x 16 4.38 | 3.91. Beyond the line the waves cover each other and the batch
+// only adds work: 200 x 16 waves 6.95 | 7.38.
+constexpr int kAdjBatch = 4;
+constexpr unsigned kAdjBatchWaves = 2048;
+
 template <int MODEL>
 int launch_adjoint(const AdjointArgs &a, int n_mid, int storage, bool polish, hipStream_t stream) {
     constexpr int AW = adj_waves<MODEL>(), kAdjThreads = AW * kWave;
@@ -630,12 +689,22 @@ int launch_adjoint(const AdjointArgs &a, int n_mid, int storage, bool polish, hi
     int rc = dispatch_storage(storage, [&](auto S) {
         dispatch_window(a.e.w, fast_index_verified(a.e.dt, a.e.tau, stream), [&](auto Wc) {
             constexpr int WW = decltype(Wc)::value, SS = decltype(S)::value;
-            if (polish)
-                hipLaunchKernelGGL((polish_kernel<MODEL, WW, SS>), dim3(blocks), dim3(kAdjThreads), 0,
-                                   stream, a);
-            else
-                hipLaunchKernelGGL((gradient_kernel<MODEL, WW, SS>), dim3(blocks), dim3(kAdjThreads),
-                                   0, stream, a);
+            auto launch = [&](auto B) {
+                constexpr int BB = decltype(B)::value;
+                if (polish)
+                    hipLaunchKernelGGL((polish_kernel<MODEL, WW, SS, BB>), dim3(blocks),
+                                       dim3(kAdjThreads), 0, stream, a);
+                else
+                    hipLaunchKernelGGL((gradient_kernel<MODEL, WW, SS, BB>), dim3(blocks),
+                                       dim3(kAdjThreads), 0, stream, a);
+            };
+            if constexpr (WW > 0 && MODEL != HSS_OCT) {
+                if (blocks <= kAdjBatchWaves && a.e.ns > a.e.w) {
+                    launch(std::integral_constant<int, WW <= 15 ? kAdjBatch : kAdjBatch / 2>{});
+                    return;
+                }
+            }
+            launch(std::integral_constant<int, 1>{});
         });
     });
     if (rc != HSS_OK) return rc;
