@@ -204,8 +204,8 @@ int hss_grid_semblance(const hss_traces *traces, const hss_midpoints *mids, int 
             default: return launch_grid_oct(la, slots, variant, traces->storage, sh.cpl, st);
         }
     };
-    if (!grid_shape_pinned(model, traces->w, variant, traces->storage) &&
-        spread_wanted(model, traces->storage, (long long)mids->n * a.ntiles)) {
+    const bool pinned = grid_shape_pinned(model, traces->w, variant, traces->storage);
+    if (!pinned && spread_wanted(model, traces->storage, (long long)mids->n * a.ntiles)) {
         const int tl = spread_tl(model, mids->n, traces->ns, traces->w, P);
         int status = HSS_OK;
         bool done;
@@ -228,6 +228,8 @@ int hss_grid_semblance(const hss_traces *traces, const hss_midpoints *mids, int 
     rc = tuned_grid_shape(model, traces->w, variant, traces->storage, mids->n, a.ntiles, st,
                           [&](GridShape sh, int slots) { return run(probe, sh, slots); }, &shape);
     if (rc != HSS_OK) return rc;
+    if (!pinned && shape.staged && staged_one_candidate(traces->w, traces->storage, P))
+        shape.cpl = 1;
     return run(a, shape, mids->n);
 }
 

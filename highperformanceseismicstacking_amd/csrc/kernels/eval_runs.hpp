@@ -113,8 +113,8 @@ __device__ __forceinline__ OctKept oct_kept_range(const OctRuns &r, int beg, int
     for (int bit = 1 << (31 - __builtin_clz(end - beg)); bit > 0; bit >>= 1) {
         const float dl = r.trace[min(k.lo + bit, end) - 1].m - om.mh;
         const float dh = r.trace[min(k.hi + bit, end) - 1].m - om.mh;
-        k.lo += (k.lo + bit <= end) & (dl < -apm) ? bit : 0;
-        k.hi += (k.hi + bit <= end) & !(dh > apm) ? bit : 0;
+        k.lo += ((k.lo + bit <= end) & (dl < -apm)) ? bit : 0;
+        k.hi += ((k.hi + bit <= end) & !(dh > apm)) ? bit : 0;
     }
     if (om.bad | !on) k.hi = k.lo;
     return k;

@@ -8,13 +8,15 @@
 // of them on 256 CUs, and a workgroup of a large launch runs long enough to leave a tail.
 // With T down to 4 a gather fills the chip, and a line's launch ends evenly.  Candidates of
 // one lane group are neighbours, so windows stay close together where T is small.  Measured
-// (T in brackets; before -> here): one 60-trace gather, 256 candidates [4] 425 -> 51 us (the
-// staged kernel); ZO-CRS, 24 midpoints, BF16 [16] 119 -> 39.9 ms, 200 midpoints 97 -> 82 ms;
+// (T in brackets; before -> here): one 60-trace gather of 640 samples, 300 candidates [4]
+// 1.13 ms -> 69 us, 90 candidates [8] 370 -> 46 us; ZO-CRS, 24 midpoints, BF16 [16] 119 -> 39.9 ms, 200 midpoints 97 -> 82 ms;
 // OCT, 30 midpoints, FP16 [4] 188 -> 48 ms (76 without the slopes' order below), 250 midpoints
-// 204 -> 101 ms; OCT, 30 midpoints in the reference's order, EXACT 105 -> 60 ms.  What bounds it then is VALU issue:
-// the 16-bit lanes widen and scale every sample of their own windows, the price of not sharing
+// 204 -> 101 ms; OCT, 30 midpoints in the reference's order, EXACT 105 -> 60 ms.
+// What bounds it then is VALU issue: the 16-bit lanes widen and scale every sample of their own windows, the price of not sharing
 // LDS segments.
 #pragma once
+
+#include <algorithm>
 
 #include "eval_lanes.hpp"
 #include "grid_impl.hpp"
@@ -86,7 +88,8 @@ __attribute__((amdgpu_waves_per_eu(spread_min_waves<MODEL, W>(), 8))) void grid_
         const int sl = rank / per_slope;
         return (rank - sl * per_slope) * period + sl;
     };
-    for (int r0 = 0; r0 < a.P; r0 += groups * CPL) {
+    // (a wave whose lanes have no candidate left ends its rounds)
+    for (int r0 = 0; r0 + wave * per_wave * CPL < a.P; r0 += groups * CPL) {
         const int q0 = r0 + grp * CPL;
         Candidate k[CPL];
         bool on[CPL];
@@ -159,28 +162,51 @@ __attribute__((amdgpu_waves_per_eu(spread_min_waves<MODEL, W>(), 8))) void grid_
     }
 }
 
-// log2 of T.  The workgroups should outnumber the CUs eight times, for a launch that ends
-// evenly; below that T halves down to 4.  T also stays at 512*CPL/P or above, where one
-// round takes all P candidates (64 candidates on 12 midpoints: T = 16 190 us, T = 8, half of the
-// lanes idle, 270 us).  T = 16 is the largest that pays (ZO-CRS, 100 midpoints: 51/45/41.9/
-// 41.4 ms at 64/32/16/8), 4 for OCT (30 midpoints, 1024 candidates: 56/50.4/48.2 ms at 16/8/4),
-// where a wave of few samples and many candidates of one slope keeps few traces of a run.
-constexpr int kSpreadWorkgroups = 2048;
+// log2 of T, 2 to 6: the one of least cost, counted in tenths of a wave's pass over a list
+// (64 samples x candidates times CPL).
+//  - Work: the passes of all waves.  A workgroup whose candidates fill few of its waves holds
+//    its slot on a CU all the same, about 3.4 passes a round (CMP, 74 midpoints, 36 candidates:
+//    0.750/0.413/0.266/0.244/0.265 ms for T = 4 to 64); an OCT workgroup spends 4.2 passes on
+//    its run list.
+//  - Passes of different T cost differently: for ZO-CRS 51/45/41.9/41.4 ms at 64/32/16/8 (100
+//    midpoints), for OCT, where a wave of few samples and many candidates of one slope keeps
+//    few traces of a run, 56/50.4/48.2 ms at 16/8/4 (30 midpoints, 1024 candidates).
+//  - Latency: rounds follow each other, some 25 us each where the chip is idle, about what
+//    1200 passes take when it is not (CMP, one midpoint, 300 candidates: 0.068/0.094/0.149/
+//    0.251/0.487 ms for T = 4 to 64).
+// Against T from the number of workgroups alone: CMP, one midpoint, 90 candidates 0.098 ->
+// 0.046 ms, 8 midpoints, 40 candidates 0.094 -> 0.052; ZO-CRS, 4 midpoints, 36 candidates
+// 1.13 -> 0.43; OCT, 16 midpoints, 32 candidates 1.51 -> 0.81; 144 candidates 3.13 -> 3.63.
 inline int spread_tl(int model, int n_slots, int ns, int w, int P) {
-    int tl = model == HSS_OCT ? 2 : 4;
-    while (tl > 2 && (long long)n_slots * ((ns + (1 << tl) - 1) >> tl) < kSpreadWorkgroups) --tl;
-    while (tl < 6 && ((long long)(2 * kSpreadThreads * spread_cpl(w)) >> tl) > P) ++tl;
+    static constexpr int kPassCost[3][5] = {
+        {108, 106, 104, 102, 100}, {105, 99, 100, 107, 122}, {100, 111, 127, 145, 170}};
+    const int *cost = kPassCost[model == HSS_CMP ? 0 : (model == HSS_ZOCRS ? 1 : 2)];
+    int tl = 2;
+    double least = 0.0;
+    for (int t = 2; t <= 6; ++t) {
+        const int per_wave = (kWave >> t) * spread_cpl(w);
+        const double waves = (double)((P - 1) / per_wave + 1);
+        const double rounds = (double)((P - 1) / (per_wave * kSpreadWaves) + 1);
+        const double wgs = (double)n_slots * (double)((ns + (1 << t) - 1) >> t);
+        const double passes = model == HSS_OCT ? waves + 4.2 : std::max(waves, 3.4 * rounds);
+        const double c = wgs * passes * cost[t - 2] + 120000.0 * rounds;
+        if (t == 2 || c < least) {
+            least = c;
+            tl = t;
+        }
+    }
     return tl;
 }
 
 // Whether a launch takes this kernel when no shape is pinned for it: ZO-CRS and OCT always
 // (measured faster at every size, above), CMP below the size where the staged kernel, which
-// reads and widens a sample once for many windows, has enough workgroups (FP32, w = 11, 512
-// candidates: 288 workgroups of it 1.62 against 1.19 ms, 600 2.17 against 2.08, 1200 3.70
-// against 3.80; FP16, w = 15: 288 1.93 against 2.08, 1200 4.45 against 6.5).
+// reads and widens a sample once for many windows, has enough workgroups (640 samples, staged
+// | spread, in ms: FP32, 250 tiles, 11 samples P = 90 0.188 | 0.170, P = 300 0.512 | 0.453,
+// 15 samples P = 300 0.590 | 0.588; 500 tiles, 11 samples P = 90 0.272 | 0.302, P = 300
+// 0.800 | 0.833; FP16, 15 samples, 80 tiles P = 300 0.526 | 0.284, 250 tiles 0.581 | 0.727).
 inline bool spread_wanted(int model, int storage, long long tiles) {
     if (model != HSS_CMP) return true;
-    return tiles <= (storage == HSS_F32 ? 768 : 240);
+    return tiles <= (storage == HSS_F32 ? 320 : 160);
 }
 
 // false: this window, variant or trace length has no such kernel.

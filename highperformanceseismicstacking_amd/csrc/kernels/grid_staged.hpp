@@ -389,6 +389,19 @@ __attribute__((amdgpu_waves_per_eu(staged_min_waves<W, VARIANT, CPL>(), 8))) voi
     res[2 * ns + so] = BI >= 0 ? 2 / sqrtf(load_candidate<HSS_CMP>(a.params, BI).c) : 0.0f;
 }
 
+// Whether few candidates go one to a lane.  A round of the eight waves is eight candidates
+// then and sixteen with two, so with two P = 24 costs what 32 does.  Two are up to 12% cheaper
+// per candidate of a full round, except in 16 bits or from 13 samples on with few rounds
+// (640 samples, 60 traces, two | one, in ms: 250 midpoints, FP32, 11 samples P = 24 0.421 |
+// 0.339, 52 0.816 | 0.716, 64 0.816 | 0.815, 72 0.980 | 0.899, 128 1.454 | 1.532, 512 5.20 |
+// 5.52; FP32, 5 samples P = 64 0.543 | 0.570; FP16, 15 samples P = 28 0.683 | 0.578, 64
+// 1.098 | 0.970, 128 1.816 | 1.800, 512 6.23 | 6.42).
+inline bool staged_one_candidate(int w, int storage, int P) {
+    const int one = (P + kStagedWaves - 1) / kStagedWaves;
+    const int two = 2 * ((P + 2 * kStagedWaves - 1) / (2 * kStagedWaves));
+    return 11 * one < 10 * two || (P <= 64 && (storage != HSS_F32 || w >= 13));
+}
+
 // Host launcher: one workgroup per (launch slot, t0 tile) (a.tt must be 1).
 int launch_grid_cmp_staged(const GridArgs &a, int n_slots, int variant, int storage, int cpl,
                            hipStream_t stream);
