@@ -225,7 +225,7 @@ int hss_grid_semblance(const hss_traces *traces, const hss_midpoints *mids, int 
     GridArgs probe = a;
     probe.not_used = nullptr;
     GridShape shape{1, 1, 0};
-    rc = tuned_grid_shape(model, traces->w, variant, traces->storage, mids->n, a.ntiles, st,
+    rc = tuned_grid_shape(model, traces->w, variant, traces->storage, mids->n, a.ntiles, P, st,
                           [&](GridShape sh, int slots) { return run(probe, sh, slots); }, &shape);
     if (rc != HSS_OK) return rc;
     if (!pinned && shape.staged && staged_one_candidate(traces->w, traces->storage, P))

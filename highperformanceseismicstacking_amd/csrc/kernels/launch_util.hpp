@@ -59,7 +59,7 @@ bool grid_shape_pinned(int model, int w, int variant, int storage);
 
 // The shape for this key, tuned on the first large launch by timing launch(shape, slots)
 // for each shape on the first `slots` launch slots of the batch (tune.hip).
-int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, int ntiles,
+int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, int ntiles, int P,
                      hipStream_t stream, const std::function<int(GridShape, int)> &launch,
                      GridShape *shape_out);
 

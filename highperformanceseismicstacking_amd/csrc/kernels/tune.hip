@@ -59,9 +59,24 @@ constexpr float kTuneMargin = 0.01f;
 // workgroups a timing run covers (a leading part of the batch); the warm-up run before it
 // (code load) covers a sixteenth of that
 constexpr unsigned kTuneBlocks = 8192;
+
+// The compensated variant's shape without timing.  CMP: up to 9 samples the staged kernel with
+// two candidates, at 11 with one, where two spill; at 13 and 15, where both spill, with two
+// from nine rounds on, in FP32 only while workgroups are few.  Else one candidate with direct
+// reads.
+// Direct | here, 640 samples, 60 traces, 300 candidates, in ms: FP32, 250 midpoints, 5
+// samples 3.11 | 2.56, 9 samples 4.22 | 3.18, 11 samples 4.54 | 4.03; 16 midpoints, 9
+// samples 1.12 | 0.47; FP16, 250 midpoints, 9 samples 5.58 | 3.14, 11 samples 6.14 | 3.98, 15 samples
+// 6.90 | 5.82 (129 candidates 3.05 | 2.88); FP32, 15 samples 60 midpoints 2.09 | 1.77, but 250
+// midpoints 5.68 | 5.79 and 129 candidates 2.55 | 2.83.
+GridShape kahan_shape(int model, int w, int storage, long long tiles, int P) {
+    if (model != HSS_CMP || w < 5 || w > 15) return GridShape{1, 1, 0};
+    if (w > 11 && (P <= 128 || (storage == HSS_F32 && tiles > 768))) return GridShape{1, 1, 0};
+    return GridShape{w == 11 ? 1 : 2, 1, 1};
+}
 }  // namespace
 
-int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, int ntiles,
+int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, int ntiles, int P,
                      hipStream_t stream, const std::function<int(GridShape, int)> &launch,
                      GridShape *shape_out) {
     int dev = 0;
@@ -77,9 +92,8 @@ int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, in
     }
     // untuned launches (small, under capture, tuning off): the choice of every tuned line
     // -- two candidates per lane, for CMP with the workgroup-staged traces -- but for the
-    // compensated variant, which keeps one candidate and direct reads (its two-candidate
-    // and staged forms spill)
-    *shape_out = variant == HSS_KAHAN ? GridShape{1, 1, 0}
+    // compensated variant
+    *shape_out = variant == HSS_KAHAN ? kahan_shape(model, w, storage, (long long)n_slots * ntiles, P)
                                       : GridShape{2, 1, model == HSS_CMP ? 1 : 0};
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
