@@ -201,24 +201,6 @@ __device__ __forceinline__ void window_single(float &A0, float &den, float y0, f
 #undef HSS_WINDOW_SINGLE
 }
 
-// Two neighbouring values u0, u1 of a window whose trace scale is factored out:
-// A += sc*u, dn = fma(u, u, dn), in registers of the right parities (window_pair).
-__device__ __forceinline__ void window_pair_scaled(float &A0, float &A1, float &dn, float u0,
-                                                   float u1, float sc, int slot) {
-#define HSS_WINDOW_PAIR_SCALED(DN, SC)                                    \
-    __asm__("v_fmac_f32 %0, %5, %3\n\t"                                   \
-            "v_fmac_f32 %2, %3, %3\n\t"                                   \
-            "v_fmac_f32 %1, %5, %4\n\t"                                   \
-            "v_fmac_f32 %2, %4, %4"                                       \
-            : "+v"(A0), "+v"(A1), "+{" DN "}"(dn)                         \
-            : "{v3}"(u0), "{v5}"(u1), "{" SC "}"(sc))
-    if (slot == 0)
-        HSS_WINDOW_PAIR_SCALED("v6", "v10");
-    else
-        HSS_WINDOW_PAIR_SCALED("v8", "v12");
-#undef HSS_WINDOW_PAIR_SCALED
-}
-
 template <int W, int VARIANT>
 struct Window {
     static constexpr int N = W > 0 ? W : kMaxWindow;
@@ -357,17 +339,16 @@ struct Window {
     }
 
     // A window's values value(0) .. value(W-1) without their trace's scale: A_j += sc*u_j and
-    // dn = sum_j u_j^2.
+    // dn = sum_j u_j^2.  Left to the compiler: the values come from conversions or mixed FMAs
+    // of four cycles each, and sums in fixed registers held their scheduling back (FP16, CMP
+    // stretch-free of 1000 midpoints, w = 15, 8.49 ms fixed, 7.28 here; ZO-CRS DE, 32 midpoints,
+    // 49.4 and 42.9 ms).
     template <class Value>
-    __device__ __forceinline__ void sum_scaled(const Value &value, float &dn, float sc, int slot) {
+    __device__ __forceinline__ void sum_scaled(const Value &value, float &dn, float sc) {
 #pragma unroll
-        for (int j = 0; j + 1 < W; j += 2) {
-            const float u0 = value(j), u1 = value(j + 1);
-            window_pair_scaled(A[j], A[j + 1], dn, u0, u1, sc, slot);
-        }
-        if constexpr (W & 1) {
-            const float u = value(W - 1);
-            A[W - 1] = __builtin_fmaf(sc, u, A[W - 1]);
+        for (int j = 0; j < W; ++j) {
+            const float u = value(j);
+            A[j] = __builtin_fmaf(sc, u, A[j]);
             dn = __builtin_fmaf(u, u, dn);
         }
     }
@@ -400,7 +381,7 @@ struct Window {
                 const float d = __builtin_fmaf((float)h[j + 1], one, -(float)h[j]);
                 return __builtin_fmaf(d, f, (float)h[j]);
             };
-            sum_scaled(value, dn, sc, slot);
+            sum_scaled(value, dn, sc);
             den = __builtin_fmaf(sc * sc, dn, den);
             used++;
             return;
@@ -420,8 +401,7 @@ struct Window {
             // the trace's scale factored out of the window: u = sc * (y0 + frac*(y1 - y0))
             // on the stored values, A_j += sc*u and den += sc^2 * sum_j u^2
             float dn = 0.0f;
-            sum_scaled([&](int j) { return __builtin_fmaf(y[j + 1] - y[j], f, y[j]); }, dn, sc,
-                       slot);
+            sum_scaled([&](int j) { return __builtin_fmaf(y[j + 1] - y[j], f, y[j]); }, dn, sc);
             den = __builtin_fmaf(sc * sc, dn, den);
         } else {
             if constexpr (FACTORED) {
