@@ -5,6 +5,10 @@
 // (t0, candidate), and selectBestSemblancesFor<Model> (cmp/linear_search.cu:83-115 and
 // twins) scans the candidates of each t0 for the first strict maximum.
 //
+// What runs here: pinned and timed launch shapes without the staged traces, HSS_KAHAN windows
+// that the staged kernel spills, and windows with no compiled form; grid_spread.hpp and
+// grid_staged.hpp take the rest.
+//
 // MI355X mapping: one workgroup = (midpoint, tile of 64 consecutive t0 samples), four
 // wavefronts.  Lane l of every wave owns t0 sample tile*64 + l; wave v evaluates
 // candidates v, v+4, v+8, ... in increasing order.  The candidate is wave-uniform (its
@@ -104,15 +108,19 @@ constexpr int grid_min_waves() { return VARIANT == HSS_KAHAN && CPL == 1 ? 7 : 1
 // The grid kernel's budget: OCT, which holds both trace loops (with and without the kept
 // offset terms), at five waves per SIMD -- the loop without them fits as before (93
 // registers), the one with them spills a few run-level values; at the compiler's own
-// choice (107 registers, four waves) the reference-order line ran 6% slower.
-template <int MODEL, int VARIANT, int CPL>
+// choice (107 registers, four waves) the reference-order line ran 6% slower.  CMP's
+// compensated windows above 9 samples spill at seven waves since their sums are written out
+// (w = 15, 16 bits: 35 registers); five waves hold them (250 midpoints, 300 candidates,
+// FP16, w = 15, 7/6/5 waves 7.23/6.27/6.24 ms, FP32 6.08/5.32/5.00, w = 11 4.30/4.01/3.94).
+template <int MODEL, int W, int VARIANT, int CPL>
 constexpr int grid_waves_budget() {
+    if (MODEL == HSS_CMP && VARIANT == HSS_KAHAN && W > 9 && CPL == 1) return 5;
     return MODEL == HSS_OCT && VARIANT != HSS_KAHAN ? 5 : grid_min_waves<VARIANT, CPL>();
 }
 
 template <int MODEL, int W, int VARIANT, int STORAGE, int CPL>
 __global__ __launch_bounds__(kGridThreads)
-__attribute__((amdgpu_waves_per_eu(grid_waves_budget<MODEL, VARIANT, CPL>(), 8))) void grid_semblance_kernel(
+__attribute__((amdgpu_waves_per_eu(grid_waves_budget<MODEL, W, VARIANT, CPL>(), 8))) void grid_semblance_kernel(
     GridArgs a) {
     constexpr int NP = MODEL == HSS_CMP ? 1 : (MODEL == HSS_ZOCRS ? 3 : 2);
     const int lane = threadIdx.x & (kWave - 1);
