@@ -25,35 +25,28 @@
 
 namespace hss {
 
-// Launch shape, chosen by timing a ZO-CRS line (200 midpoints, ~930 traces each, NP 32,
-// G 50, BF16) and an OCT line (300 midpoints, ~2150 traces each, NP 48, G 40, FP16):
-//  * de_cpl: individuals per lane in one trace loop.  Two interleave two independent
-//    traveltime/window chains, which hides the latency of the long dependent OCT and
-//    ZO-CRS sequences better than more resident waves do (OCT -10%, ZO-CRS -6%; three
-//    were slower for ZO-CRS and no better for OCT).
-//  * de_min_occupancy: the register budget, as waves per SIMD the compiler must fit
-//    (OCT 6: 80 VGPRs; ZO-CRS 8: 64; CMP 8: 64).  Since the traveltime terms are kept
-//    across traces (offset groups, midpoint runs) the trace loop is short and waits on
-//    memory, and more resident waves pay for the spills of the per-generation code:
-//    OCT 5/6/7/8 waves measured 2435/2334/2356/2479 ms, ZO-CRS 6/7/8 559/557/536 ms.
-//  * de_waves: waves per workgroup, so that whole workgroups fill a CU's wave slots at
-//    that occupancy (OCT 8 x 3 workgroups = 24 per CU; ZO-CRS and CMP 8 x 4 = 32).  For OCT
-//    8 waves were 1.4% faster than 4 x 6 workgroups: a workgroup's generations run half as
-//    long, so the launch's tail (the last workgroups on each XCD, about a quarter of a
-//    second each at 4 waves) is shorter.
-// Kahan windows (twice the accumulators), windows above 11 samples and the runtime-w
-// kernel keep one individual per lane and the compiler's own register budget.
+// Launch shape of de_semblance_kernel, which runs large ZO-CRS launches and every model's
+// compensated and non-compiled windows (de_spread_kernel below takes the rest), chosen by
+// timing a ZO-CRS line (200 midpoints, ~930 traces each, NP 32, G 50, BF16).  ZO-CRS with a
+// compiled window of up to 11 samples:
+//  * de_cpl: two individuals per lane in one trace loop interleave two independent
+//    traveltime/window chains, which hides their latency better than more resident waves
+//    do (-6%; three were slower);
+//  * de_min_occupancy: eight waves per SIMD, 64 VGPRs: the traveltime terms are kept across
+//    a midpoint's traces, the trace loop is short and waits on memory, and more resident
+//    waves pay for the spills of the per-generation code (6/7/8 waves 559/557/536 ms);
+//  * de_waves: eight waves, so that four whole workgroups fill a CU's wave slots.
+// The others keep one individual per lane and the compiler's own register budget.
 template <int MODEL>
 constexpr int de_waves() { return 8; }
 template <int MODEL, int W, int VARIANT>
-constexpr bool de_tuned() { return VARIANT != HSS_KAHAN && W != 0 && W <= 11; }
-template <int MODEL, int W, int VARIANT>
-constexpr int de_cpl() { return de_tuned<MODEL, W, VARIANT>() && MODEL != HSS_CMP ? 2 : 1; }
-template <int MODEL, int W, int VARIANT>
-constexpr int de_min_occupancy() {
-    if (!de_tuned<MODEL, W, VARIANT>()) return 1;
-    return MODEL == HSS_OCT ? 6 : 8;
+constexpr bool de_tuned() {
+    return MODEL == HSS_ZOCRS && VARIANT != HSS_KAHAN && W != 0 && W <= 11;
 }
+template <int MODEL, int W, int VARIANT>
+constexpr int de_cpl() { return de_tuned<MODEL, W, VARIANT>() ? 2 : 1; }
+template <int MODEL, int W, int VARIANT>
+constexpr int de_min_occupancy() { return de_tuned<MODEL, W, VARIANT>() ? 8 : 1; }
 constexpr int kDeWavesMax = 8;
 // Every lane carries its own individual, so a trace's windows spread over far more than
 // one wave segment; DE reads 16-bit windows per lane (Window::add16) instead.
@@ -61,8 +54,7 @@ constexpr bool kDeSegments = false;
 // OCT: DE keeps the offset-dependent half of the traveltime across consecutive traces
 // with the same half offset (the host layer groups the lists of the non-exact variants by
 // offset).  Any order gives the bits of computing every trace afresh; in the reference's
-// (m, h) order, where nothing is shared, the launch is about 11% slower than a kernel that
-// does not keep them (measured on the C4 line).
+// (m, h) order nothing is shared.
 constexpr bool kDeOctKeep = true;
 // OCT: the aperture test of a run of traces first, then each lane's kept traces only
 // (eval_compact.hpp); same bits as evaluate_n.  Not for HSS_KAHAN.

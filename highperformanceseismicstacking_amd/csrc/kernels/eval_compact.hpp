@@ -1,4 +1,6 @@
-// OCT evaluation with compacted trace passes, for the differential-evolution kernel.
+// OCT evaluation with compacted trace passes, for the kernels whose lanes carry candidates of
+// their own, on lists that eval_runs.hpp's walk does not take (more traces or offset runs than
+// it holds in LDS, or midpoints unsorted inside a run).
 //
 // In an OCT evaluation most traces fall outside the aperture |m - mh| <= apm around the
 // candidate's displaced midpoint mh (about three in four on a line whose selected traces
