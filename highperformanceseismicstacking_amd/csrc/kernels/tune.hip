@@ -64,11 +64,10 @@ constexpr unsigned kTuneBlocks = 8192;
 // two candidates, at 11 with one, where two spill; at 13 and 15, where both spill, with two
 // from nine rounds on, in FP32 only while workgroups are few.  Else one candidate with direct
 // reads.
-// Direct | here, 640 samples, 60 traces, 300 candidates, in ms: FP32, 250 midpoints, 5
-// samples 3.11 | 2.56, 9 samples 4.22 | 3.18, 11 samples 4.54 | 4.03; 16 midpoints, 9
-// samples 1.12 | 0.47; FP16, 250 midpoints, 9 samples 5.58 | 3.14, 11 samples 6.14 | 3.98, 15 samples
-// 6.90 | 5.82 (129 candidates 3.05 | 2.88); FP32, 15 samples 60 midpoints 2.09 | 1.77, but 250
-// midpoints 5.68 | 5.79 and 129 candidates 2.55 | 2.83.
+// Direct | staged, 640 samples, 60 traces, 300 candidates, in ms: FP32, 250 midpoints, 5
+// samples 3.11 | 2.56, 9 samples 4.22 | 3.18, 11 samples 3.94 | 4.03, 15 samples 5.00 | 5.79;
+// 16 midpoints, 9 samples 1.12 | 0.47, 11 samples 1.02 | 0.72, 15 samples 1.15 | 0.63; FP16,
+// 250 midpoints, 9 samples 5.58 | 3.14, 11 samples 5.32 | 3.98, 15 samples 6.24 | 5.82.
 GridShape kahan_shape(int model, int w, int storage, long long tiles, int P) {
     if (model != HSS_CMP || w < 5 || w > 15) return GridShape{1, 1, 0};
     if (w > 11 && (P <= 128 || (storage == HSS_F32 && tiles > 768))) return GridShape{1, 1, 0};
