@@ -405,9 +405,9 @@ __device__ __forceinline__ bool oct_traveltime_at(const OctMid &d, const OctTime
 // NaN fails both compares.  index_bounds() computes (lo, hi) on the host; ns < 2^24
 // keeps hi exact.
 // FAST (tau >= 1) makes the test on the index: tau <= k < K as one unsigned comparison,
-// k - tau < span = max(K - tau, 0), of a value the window's address needs anyway.  The
-// conversion gives 0 for a NaN and saturates, both outside; ZO-CRS differential evolution,
-// 32 midpoints, 92.6 -> 90.6 ms against the two float comparisons.
+// k - tau < span = max(K - tau, 0), of a value the window's address needs anyway.  A NaN's
+// index is 0 and one out of int range saturates (sample_index), both outside; ZO-CRS
+// differential evolution, 32 midpoints, 92.6 -> 90.6 ms against the two float comparisons.
 struct IndexBounds {
     float lo, hi;
     int tau, span;
@@ -423,15 +423,30 @@ __host__ __device__ inline IndexBounds index_bounds(int ns, int tau) {
     return b;
 }
 
+// t/dt truncated to an int, for every float: v_cvt_i32_f32 gives 0 for a NaN and the nearest
+// int for a value out of int range.  A C++ conversion of such a value is undefined, and the
+// compiler may take whatever follows from it, the window test included, as it likes; its
+// own saturating form (-fno-strict-float-cast-overflow) adds three compares and selects.
+__device__ __forceinline__ int sample_index(float ti) {
+    int k;
+    __asm__("v_cvt_i32_f32 %0, %1" : "=v"(k) : "v"(ti));
+    return k;
+}
+
+// k - tau, wrapping where k is the smallest int.
+__device__ __forceinline__ int window_first(int k, int tau) {
+    return (int)((unsigned)k - (unsigned)tau);
+}
+
 template <bool FAST = false>
 __device__ __forceinline__ bool window_index(float t, float dt, float inv, IndexBounds ib,
                                              int tau, int *first, float *frac) {
     float ti;
     if constexpr (FAST) ti = div_rn(t, dt, inv);
     else ti = t / dt;
-    const int k = (int)ti;
+    const int k = sample_index(ti);
     *frac = ti - (float)k;
-    *first = k - tau;
+    *first = window_first(k, tau);
     return ti > ib.lo && ti < ib.hi;
 }
 
@@ -445,11 +460,11 @@ __device__ __forceinline__ bool window_k(float t, float dt, float inv, IndexBoun
     float ti;
     if constexpr (FAST) ti = div_rn(t, dt, inv);
     else ti = t / dt;
-    const int k = (int)ti;
+    const int k = sample_index(ti);
     if constexpr (FAST) *frac = __builtin_amdgcn_fractf(ti);
     else *frac = ti - (float)k;
     *k_out = k;
-    if constexpr (FAST) return (unsigned)(k - ib.tau) < (unsigned)ib.span;
+    if constexpr (FAST) return (unsigned)window_first(k, ib.tau) < (unsigned)ib.span;
     return ti > ib.lo && ti < ib.hi;
 }
 

@@ -12,6 +12,9 @@
 // index, t/dt - (float)(int)(t/dt), is taken as v_fract_f32(t/dt); that too is compared
 // for every float in [1, 2^24).  The launchers use the short sequences only for tau >= 1.
 // One launch walks all 2^32 bit patterns; the result is cached per (device, dt).
+//
+// hss_verify_index_ops also compares window_k's test on the index with the two float
+// comparisons it stands for, on every bit pattern (NaNs and infinities among them) as t/dt.
 #include <map>
 #include <mutex>
 #include <utility>
@@ -23,11 +26,29 @@ namespace hss {
 
 __device__ unsigned long long verify_mismatches;
 
-__global__ __launch_bounds__(256) void verify_index_ops_kernel(float dt, float inv, int check_sqrt) {
+// What window_k accepts of a t/dt of `ti` (dt = 1, which leaves ti as it is, but for the
+// infinities, whose quotient is a NaN).
+__device__ __forceinline__ bool index_test_differs(float ti, IndexBounds ib) {
+    int k;
+    float f;
+    const bool in = window_k<true>(ti, 1.0f, 1.0f, ib, &k, &f);
+    return in != (ti > ib.lo && ti < ib.hi) || (in && k != (int)ti);
+}
+
+// The window bounds to put through index_test_differs.
+struct WindowChecks {
+    int n;
+    IndexBounds ib[4];
+};
+
+__global__ __launch_bounds__(256) void verify_index_ops_kernel(float dt, float inv, int check_sqrt,
+                                                                  WindowChecks windows) {
     unsigned long long bad = 0;
     const unsigned stride = gridDim.x * blockDim.x;
     for (unsigned long long b = blockIdx.x * blockDim.x + threadIdx.x; b < (1ull << 32); b += stride) {
         const float x = __uint_as_float((unsigned)b);
+        for (int i = 0; i < windows.n; ++i)
+            if (index_test_differs(x, windows.ib[i])) bad++;
         if (x != x) continue;  // NaN inputs never reach either sequence
         if (check_sqrt) {
             // same bits for x >= 0 (and -0); a NaN for x < 0, as sqrtf gives
@@ -83,7 +104,8 @@ bool fast_index_verified(float dt, int tau, hipStream_t stream) {
     if (hipMemcpyToSymbolAsync(HIP_SYMBOL(verify_mismatches), &zero, sizeof(zero), 0,
                                hipMemcpyHostToDevice, stream) != hipSuccess)
         return false;
-    hipLaunchKernelGGL(verify_index_ops_kernel, dim3(8192), dim3(256), 0, stream, dt, inv, 1);
+    hipLaunchKernelGGL(verify_index_ops_kernel, dim3(8192), dim3(256), 0, stream, dt, inv, 1,
+                       WindowChecks{});
     if (hipGetLastError() != hipSuccess ||
         hipMemcpyFromSymbolAsync(&bad, HIP_SYMBOL(verify_mismatches), sizeof(bad), 0,
                                  hipMemcpyDeviceToHost, stream) != hipSuccess ||
@@ -118,7 +140,11 @@ extern "C" int hss_verify_index_ops(float dt, unsigned long long *mismatches, vo
     hipError_t e = hipMemcpyToSymbolAsync(HIP_SYMBOL(verify_mismatches), &zero, sizeof(zero), 0,
                                           hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(verify_index_ops_kernel, dim3(8192), dim3(256), 0, st, dt, 1.0f / dt, 1);
+    // a trace with two windows, an ordinary one, one too short, a very long one
+    const WindowChecks windows{4, {index_bounds(33, 15), index_bounds(2001, 5),
+                                   index_bounds(31, 15), index_bounds((1 << 24) - 1, 1)}};
+    hipLaunchKernelGGL(verify_index_ops_kernel, dim3(8192), dim3(256), 0, st, dt, 1.0f / dt, 1,
+                       windows);
     e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     e = hipMemcpyFromSymbolAsync(mismatches, HIP_SYMBOL(verify_mismatches), sizeof(*mismatches), 0,
