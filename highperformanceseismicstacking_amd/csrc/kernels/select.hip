@@ -87,7 +87,8 @@ __device__ __forceinline__ void oct_candidate(const SelectArgs &a, int g, int s,
 // kBins/rows bins over [-sqrt(h^2+h0^2), +sqrt(h^2+h0^2)], each with the smallest and largest
 // displacement in it.  A trace then looks at the few bins its interval reaches: the exact
 // test at a bin's two ends answers for the whole bin unless the interval lies strictly
-// between them (an aperture narrower than a bin), where the trace tests the slice itself.
+// between them (an aperture narrower than a bin): the pairs of trace and midpoint left open
+// so are tested against the slice's displacements one by one (select_oct_scan).
 // The slices only ever set mask bytes that a first launch cleared, so they need not know of
 // each other.
 //
@@ -109,7 +110,7 @@ constexpr int kSlots = 2 * kOffsetsMax;  // open-addressed table of the block's 
 constexpr int kOctThreads = 1024;
 constexpr int kTracesPerThread = 4;
 constexpr int kBlockTraces = kOctThreads * kTracesPerThread;
-constexpr int kPairMidpoints = 64;       // midpoints of a group in pairs mode
+constexpr int kPairMidpoints = 64;       // midpoints of a group in pairs mode (bits of a word)
 
 // Floats as unsigned integers of the same order.
 __device__ __forceinline__ uint32_t order_key(float x) {
@@ -125,7 +126,12 @@ struct OctRows {
     int number[kSlots];  // the offset's number; row = number - the pass's first
     float h[kOffsetsMax];
     float low[kRowsMax], per_unit[kRowsMax];  // the bins' start and bins per unit of d
-    uint32_t least[kBins], most[kBins];       // order keys; least > most: empty
+    union {
+        struct {
+            uint32_t least[kBins], most[kBins];  // order keys; least > most: empty
+        };
+        float scan[2 * kBins];  // select_oct_scan: rows of displacements
+    };
     unsigned long long filled[kBins / 64];    // bit b of word w: bin 64*w + b is not empty
     int n;
 };
@@ -148,22 +154,49 @@ __device__ __forceinline__ int oct_side(float m, float m0, float d, float apm) {
     return x > apm ? 1 : (x < -apm ? -1 : 2);
 }
 
-// Whether some displacement of the slice [qa, qb) passes, one by one.
-__device__ bool oct_test_slice(const SelectArgs &a, int g, float m, float h, float m0, int NP,
-                               long long qa, long long qb) {
-    int s = (int)(qa / NP), p = (int)(qa - (long long)s * NP);
-    for (long long q = qa; q < qb; ++q) {
-        float c, slope, d;
-        oct_candidate(a, g, s, p, &c, &slope);
-        if (oct_displacement(h, a.h0, (float)s * a.dt, c, slope, &d) == kNoError &&
-            oct_side(m, m0, d, a.apm) == 0)
-            return true;
-        if (++p == NP) {
-            p = 0;
-            ++s;
+// The exact test of (trace, midpoint) pairs the bins leave open: bit g of unsure[j] is midpoint
+// g0 + g of trace i0 + kOctThreads*j + tid.  The slice's displacements are worked out a chunk at
+// a time into LDS, once per row, and every open pair looks at every one of its row's: 30
+// midpoints x 4832 traces, 1024 pairs, apertures of 2/1/0 m 10/20/57 ms.  (376/533/632 ms when
+// each open pair worked the displacements out for itself, 138/161/185 ms in the kernel before
+// the bins.)
+__device__ void select_oct_scan(const SelectArgs &a, OctRows &t, int i0, int g0, int first,
+                                int rows, int NP, long long qa, long long qb,
+                                unsigned long long (&unsure)[kTracesPerThread]) {
+    const int tid = (int)threadIdx.x;
+    // a row of the table has an odd length: the lanes of a wave read one place of many rows
+    const int stride = (2 * kBins / rows - 1) | 1, chunk = stride - 1;
+    for (long long q0 = qa; q0 < qb; q0 += chunk) {
+        unsigned long long open = 0;
+        for (int j = 0; j < kTracesPerThread; ++j) open |= unsure[j];
+        if (!__syncthreads_or(open != 0)) return;  // (also before the table is written again)
+        const int n = (int)min((long long)chunk, qb - q0);
+        for (int k = tid; k < n * rows; k += kOctThreads) {
+            const int row = k / n, at = k - row * n;
+            const int s = (int)((q0 + at) / NP), p = (int)(q0 + at - (long long)s * NP);
+            float c, slope, d;
+            oct_candidate(a, g0, s, p, &c, &slope);
+            const int err = oct_displacement(t.h[first + row], a.h0, (float)s * a.dt, c, slope, &d);
+            t.scan[row * stride + at] = err == kNoError ? d : __int_as_float(0x7fc00000);
+        }
+        __syncthreads();
+        for (int j = 0; j < kTracesPerThread; ++j) {
+            if (unsure[j] == 0) continue;
+            const int i = i0 + j * kOctThreads + tid;
+            const float m = a.mid[i];
+            const int row = t.number[offset_slot(t, __float_as_uint(a.hoff[i]))] - first;
+            const float *d = t.scan + row * stride;
+            for (unsigned long long rest = unsure[j]; rest != 0; rest &= rest - 1) {
+                const int g = g0 + __builtin_ctzll(rest);
+                const float m0 = a.m0[g];
+                bool used = false;
+                for (int k = 0; k < n; ++k) used |= oct_side(m, m0, d[k], a.apm) == 0;
+                if (!used) continue;
+                a.mask[(size_t)g * a.ntr + i] = 1;
+                unsure[j] &= ~(rest & -rest);
+            }
         }
     }
-    return false;
 }
 
 // Every trace of the block tests the slice's candidates, kOctThreads of them at a time, which
@@ -317,7 +350,9 @@ __global__ __launch_bounds__(kOctThreads) void select_oct_kernel(SelectArgs a, i
         }
         __syncthreads();
 
+        unsigned long long left[kTracesPerThread];  // bit g - g0: the bins do not answer
         for (int j = 0; j < kTracesPerThread; ++j) {
+            left[j] = 0;
             if (!((reached >> j) & 1)) continue;
             const int i = i0 + j * kOctThreads + tid;
             const float m = a.mid[i], h = a.hoff[i];
@@ -348,10 +383,13 @@ __global__ __launch_bounds__(kOctThreads) void select_oct_kernel(SelectArgs a, i
                     used = lo == 0 || hi == 0;
                     unsure = unsure || lo != hi;
                 }
-                if (!used && unsure) used = oct_test_slice(a, g, m, h, m0, NP, qa, qb);
-                if (used) a.mask[(size_t)g * a.ntr + i] = 1;
+                if (used)
+                    a.mask[(size_t)g * a.ntr + i] = 1;
+                else if (unsure)
+                    left[j] |= 1ull << (g - g0);
             }
         }
+        select_oct_scan(a, t, i0, g0, first, rows, NP, qa, qb, left);
         __syncthreads();  // the bins are cleared next
     }
 }
