@@ -18,6 +18,8 @@
 // coalesced row; one workgroup barrier separates generations.
 #pragma once
 
+#include <cstddef>
+
 #include "eval_compact.hpp"
 #include "eval_runs.hpp"
 #include "grid_impl.hpp"
@@ -411,10 +413,24 @@ __attribute__((amdgpu_waves_per_eu(6, 8))) void de_spread_kernel(DeArgs a) {
     auto rec = [&](int buf, int i, int f) -> float * {
         return column + ((size_t)(buf * NP + i) * REC + f) * kWave;
     };
-    __shared__ std::conditional_t<de_compact<MODEL, VARIANT>(), OctRuns, int> runs;
+    // OCT: the midpoint's offset runs, or, for lists that do not fit them, the waves' records of
+    // a chunk of traces for the compacted walk, where the list has runs at all (in the
+    // reference's order its two passes find little to skip, and evaluate_n is faster).  150
+    // midpoints, NP = 48, two generations, evaluate_n | compacted walk, in ms: grouped lists of
+    // ~3700 traces, FP16 77.7 | 62.2, ~4600, FP16 96.9 | 75.4, FP32 78.0 | 64.0; ~2400 in the
+    // reference's order, FP32 EXACT 115.8 | 124.1.
+    union OctLists {
+        OctRuns runs;
+        OctTraceRec chunk[kDeSpreadWaves][kWave];
+    };
+    static_assert(sizeof(OctLists::chunk) <= offsetof(OctRuns, n),
+                  "a wave may write its records while another still reads runs.n");
+    __shared__ std::conditional_t<de_compact<MODEL, VARIANT>(), OctLists, int> oct_lists;
     bool by_runs = false;
     if constexpr (de_compact<MODEL, VARIANT>())
-        by_runs = load_oct_runs(e, STORAGE == HSS_F32 ? 4 : 2, runs);
+        by_runs = load_oct_runs(e, STORAGE == HSS_F32 ? 4 : 2, oct_lists.runs);
+    bool compact = false;
+    if constexpr (de_compact<MODEL, VARIANT>()) compact = !by_runs && oct_offset_runs_long(e);
     uint64_t rejected = 0;  // the wave's rejections (uniform)
     auto eval = [&](const Candidate &k, bool on, float *S, float *stk) {
         const Candidate kc[1] = {k};
@@ -424,8 +440,11 @@ __attribute__((amdgpu_waves_per_eu(6, 8))) void de_spread_kernel(DeArgs a) {
         const bool live = active && on;
         if constexpr (de_compact<MODEL, VARIANT>()) {
             if (by_runs)
-                evaluate_oct_runs<W, VARIANT, STORAGE, false, 1>(e, runs, t0, kc, on1, 0.0f, live,
-                                                                 S1, T1, &rej);
+                evaluate_oct_runs<W, VARIANT, STORAGE, false, 1>(e, oct_lists.runs, t0, kc, on1,
+                                                                 0.0f, live, S1, T1, &rej);
+            else if (compact)
+                evaluate_oct_compact<W, VARIANT, STORAGE, false, 1>(
+                    e, t0, kc, on1, 0.0f, live, oct_lists.chunk[wave], S1, T1, &rej);
             else
                 evaluate_n<MODEL, W, VARIANT, STORAGE, false, 1, kDeSegments, kDeOctKeep>(
                     e, t0, t0 * t0, kc, on1, 0.0f, live, nullptr, S1, T1, &rej);
