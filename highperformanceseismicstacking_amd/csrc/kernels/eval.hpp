@@ -136,6 +136,17 @@ __device__ __forceinline__ void evaluate_n(const EvalCtx &e, float t0, float t0s
     using Reader = SampleReader<STORAGE>;
     constexpr bool USE_SEG = SEG && W > 0;
     constexpr bool FASTIDX = W != 0;
+    // HSS_KAHAN has twice the sums in registers, and with the window's samples and the fixed
+    // registers of the paired form beside them these kernels spill.  Paired | here, grid search:
+    // CMP, FP16, w = 15, 256 midpoints of 2001 samples, 512 candidates 39.6 | 36.6 ms; OCT, 12
+    // midpoints, w = 11, FP16 65.9 | 61.9, FP32 51.6 | 48.1; ZO-CRS, BF16, w = 15 24.5 | 24.1
+    // (30.7 in turn).
+    constexpr Summing HOW =
+        VARIANT != HSS_KAHAN                  ? Summing::Paired
+        : MODEL == HSS_OCT                    ? (SHIFT ? Summing::Paired : Summing::Plain)
+        : USE_SEG && MODEL == HSS_CMP         ? Summing::InTurn
+        : USE_SEG                             ? Summing::Plain
+                                              : Summing::Paired;
     const bool scaled = (STORAGE != HSS_F32) && e.scale != nullptr;
     Reader rd{(decltype(Reader::p))e.samples};
     Window<W, VARIANT> acc[CPL];
@@ -311,7 +322,8 @@ __device__ __forceinline__ void evaluate_n(const EvalCtx &e, float t0, float t0s
                     for (int c = 0; c < CPL; ++c) {
                         const int rel = kk[c] - e.tau - b + par;
                         const bool fits = (unsigned)rel <= (unsigned)(kSeg - 1 - W);
-                        if (serve[c] & fits) acc[c].add_lds(seg + rel, f[c], e.w, c);
+                        if (serve[c] & fits)
+                            acc[c].template add_lds<HOW>(seg + rel, f[c], e.w, c);
                         rest[c] = serve[c] & !fits;
                     }
                 };
@@ -343,7 +355,7 @@ __device__ __forceinline__ void evaluate_n(const EvalCtx &e, float t0, float t0s
                 const float *row = (const float *)e.samples + trace0 - (size_t)e.tau;
 #pragma unroll
                 for (int c = 0; c < CPL; ++c) {
-                    if (use[c]) acc[c].add_row(row, (unsigned)kk[c], f[c], e.w, c);
+                    if (use[c]) acc[c].template add_row<HOW>(row, (unsigned)kk[c], f[c], e.w, c);
                 }
             } else if constexpr (W > 0) {
                 // 16-bit samples, per-lane reads of whole words (add16) from the trace's

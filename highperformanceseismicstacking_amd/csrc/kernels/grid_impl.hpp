@@ -109,18 +109,20 @@ constexpr int grid_min_waves() { return VARIANT == HSS_KAHAN && CPL == 1 ? 7 : 1
 // offset terms), at five waves per SIMD -- the loop without them fits as before (93
 // registers), the one with them spills a few run-level values; at the compiler's own
 // choice (107 registers, four waves) the reference-order line ran 6% slower.  CMP's
-// compensated windows above 9 samples spill at seven waves since their sums are written out
-// (w = 15, 16 bits: 35 registers); five waves hold them (250 midpoints, 300 candidates,
-// FP16, w = 15, 7/6/5 waves 7.23/6.27/6.24 ms, FP32 6.08/5.32/5.00, w = 11 4.30/4.01/3.94).
-template <int MODEL, int W, int VARIANT, int CPL>
+// compensated FP32 windows above 9 samples hold the window beside their sums and would spill
+// at seven waves (w = 15, 256 midpoints of 2001 samples, 256 candidates 18.4 ms, five waves
+// 17.4); 16-bit ones, summed one sample after the other, fit them all but a few registers
+// (FP16, the same line, seven/six/five waves 18.7/19.7/19.9 ms).
+template <int MODEL, int W, int VARIANT, int STORAGE, int CPL>
 constexpr int grid_waves_budget() {
-    if (MODEL == HSS_CMP && VARIANT == HSS_KAHAN && W > 9 && CPL == 1) return 5;
+    if (MODEL == HSS_CMP && VARIANT == HSS_KAHAN && STORAGE == HSS_F32 && W > 9 && CPL == 1)
+        return 5;
     return MODEL == HSS_OCT && VARIANT != HSS_KAHAN ? 5 : grid_min_waves<VARIANT, CPL>();
 }
 
 template <int MODEL, int W, int VARIANT, int STORAGE, int CPL>
 __global__ __launch_bounds__(kGridThreads)
-__attribute__((amdgpu_waves_per_eu(grid_waves_budget<MODEL, W, VARIANT, CPL>(), 8))) void grid_semblance_kernel(
+__attribute__((amdgpu_waves_per_eu(grid_waves_budget<MODEL, W, VARIANT, STORAGE, CPL>(), 8))) void grid_semblance_kernel(
     GridArgs a) {
     constexpr int NP = MODEL == HSS_CMP ? 1 : (MODEL == HSS_ZOCRS ? 3 : 2);
     const int lane = threadIdx.x & (kWave - 1);

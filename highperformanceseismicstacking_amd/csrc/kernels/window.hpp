@@ -201,6 +201,12 @@ __device__ __forceinline__ void window_single(float &A0, float &den, float y0, f
 #undef HSS_WINDOW_SINGLE
 }
 
+// How a window's samples are summed; the same bits.  Paired: all of them in registers, the sums
+// in window_pair's fixed ones.  Plain: all in registers, the rest left to the compiler.  InTurn:
+// one sample after the other, for kernels whose sums take the registers.  (HSS_EXACT is never
+// Paired.)
+enum class Summing { Paired, Plain, InTurn };
+
 template <int W, int VARIANT>
 struct Window {
     static constexpr int N = W > 0 ? W : kMaxWindow;
@@ -263,10 +269,10 @@ struct Window {
     }
 
     // The window whose samples are y[0..W] (compiled window sizes).
-    template <class Samples>
+    template <Summing HOW = Summing::Paired, class Samples>
     __device__ __forceinline__ void sum(const Samples &y, float f, int slot) {
         static_assert(W > 0, "a compiled window size");
-        if constexpr (VARIANT == HSS_EXACT) {
+        if constexpr (VARIANT == HSS_EXACT || HOW != Summing::Paired) {
 #pragma unroll
             for (int j = 0; j < W; ++j) step(j, y[j], y[j + 1], f);
         } else {
@@ -277,20 +283,21 @@ struct Window {
         }
     }
 
-    // A window in LDS, row[0..W], without counting its trace in `used`.
-    __device__ __forceinline__ void sum_lds(const LdsFloat *row, float f, int w, int slot) {
-        if constexpr (W > 0) {
+    // The window that starts at p[0], without counting its trace in `used`.
+    template <Summing HOW, class Samples>
+    __device__ __forceinline__ void sum_from(Samples p, float f, int w, int slot) {
+        if constexpr (W > 0 && HOW != Summing::InTurn) {
             float y[W + 1];
 #pragma unroll
-            for (int j = 0; j <= W; ++j) y[j] = row[j];
-            sum(y, f, slot);
+            for (int j = 0; j <= W; ++j) y[j] = p[j];
+            sum<HOW>(y, f, slot);
         } else {
-            float y1 = row[0];
+            float y1 = p[0];
 #pragma unroll
             for (int j = 0; j < N; ++j) {
-                if (j >= w) continue;
+                if (W == 0 && j >= w) continue;
                 const float y0 = y1;
-                y1 = row[j + 1];
+                y1 = p[j + 1];
                 step(j, y0, y1, f);
             }
         }
@@ -316,25 +323,10 @@ struct Window {
     // FP32 samples of one trace: row[k .. k+w] with `row` wave-uniform (the trace's first
     // sample minus tau) and k the lane's sample index, so the loads take a scalar base and
     // a 32-bit lane offset.
+    template <Summing HOW = Summing::Paired>
     __device__ __forceinline__ void add_row(const float *row, unsigned k, float f, int w,
                                             int slot = 0) {
-        const float *p = row + k;
-        if constexpr (W > 0) {
-            float y[W + 1];
-#pragma unroll
-            for (int j = 0; j <= W; ++j) y[j] = p[j];
-            sum(y, f, slot);
-            used++;
-            return;
-        }
-        float y1 = p[0];
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            if (W == 0 && j >= w) continue;
-            const float y0 = y1;
-            y1 = p[j + 1];
-            step(j, y0, y1, f);
-        }
+        sum_from<HOW>(row + k, f, w, slot);
         used++;
     }
 
@@ -440,8 +432,9 @@ struct Window {
     }
 
     // Same as add() for a window already decoded (and scaled) into LDS: row[0..w].
-    __device__ __forceinline__ void add_lds(const LdsFloat *row, float f, int w, int slot = 0) {
-        sum_lds(row, f, w, slot);
+    template <Summing HOW>
+    __device__ __forceinline__ void add_lds(const LdsFloat *row, float f, int w, int slot) {
+        sum_from<HOW>(row, f, w, slot);
         used++;
     }
 
