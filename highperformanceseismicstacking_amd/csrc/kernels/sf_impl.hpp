@@ -34,8 +34,12 @@ namespace hss {
 constexpr int kSfMaxShifts = 64;
 constexpr int kSfWaves = 8;
 constexpr int kSfThreads = kSfWaves * kWave;
-// (sample, shift) pairs whose results fit the workgroup's LDS.
+// (sample, shift) pairs of a workgroup, as many as the largest shift list has in a 64-sample
+// tile: 32 KB of dynamic LDS, for OCT beside 45 KB of run lists (78 of a CU's 160 KB).
 constexpr int kSfPairs = 4096;
+static_assert(kSfPairs * sizeof(float2) + sizeof(OctRuns) + 2 * kSfMaxShifts * sizeof(int) <=
+                  160 * 1024,
+              "a workgroup's LDS");
 // Lanes read windows per lane (Window::add16 for 16-bit storage): they belong to several
 // candidates, so a trace's windows spread over more than one wave segment.
 constexpr bool kSfSegments = false;
@@ -209,13 +213,19 @@ __attribute__((amdgpu_waves_per_eu(sf_min_waves<MODEL, W, VARIANT>(), 8))) void 
 // 32/64/128/256 1.83/1.67/1.72/1.68 ms.)
 constexpr int kSfTile = 64;
 constexpr long long kSfWorkgroups = 1024;
-// The waves, five to eight, that leave the fewest idle in the last round over the pairs.
-inline int sf_waves(int pairs) {
-    const int need = (pairs + kWave - 1) / kWave;
-    int best = kSfWaves;
-    for (int w = kSfWaves - 1; w >= 5; --w)
-        if ((need + w - 1) / w * w < (need + best - 1) / best * best) best = w;
-    return std::min(best, need);
+// Waves of a workgroup: four per SIMD pair up evenly, so eight, which read one tile's windows
+// together, or four where the registers (the compensated sums above 9 samples, the runtime-w
+// kernel) leave so few waves per SIMD that whole workgroups of eight waste them, in launches
+// that fill the chip.  Five to seven, which leave fewer lanes idle in the last round over the
+// pairs, load the SIMDs unevenly: 21 shifts, seven | eight | four waves, in ms, CMP, 300
+// midpoints, FP16, w = 7 1.09 | 0.99 | 1.00, FP16, EXACT, w = 11 2.23 | 2.10 | 2.11, FP32, w = 15
+// 1.25 | 1.24 | 1.26; compensated, BF16, w = 13 1.52 | 1.41 | 1.22; ZO-CRS, BF16, w = 11, 60
+// midpoints 3.01 | 2.65 | 2.81, 400 midpoints 15.9 | 14.4 | 15.3; OCT, FP16, w = 11, 100
+// midpoints 3.2 | 3.0 | 4.8 (every workgroup reads the midpoint's list).
+template <int MODEL, int W, int VARIANT>
+constexpr int sf_waves(long long workgroups) {
+    const bool few = MODEL != HSS_OCT && (W == 0 || (VARIANT == HSS_KAHAN && W > 9));
+    return few && workgroups >= kSfWorkgroups ? 4 : kSfWaves;
 }
 inline int sf_tile(long long n_mid, int ns, int nN) {
     int tile = kSfTile;
@@ -235,17 +245,18 @@ int launch_sf(const SfArgs &args, int n_mid, int variant, int storage, hipStream
     if (blocks > 0x7fffffffull) return HSS_ERR_INVALID_SIZE;
     if (blocks == 0) return HSS_OK;
     const unsigned lds = (unsigned)(a.tile * a.nN) * sizeof(float2);
-    const unsigned threads = (unsigned)sf_waves(a.tile * a.nN) * kWave;
+    const int need = (a.tile * a.nN + kWave - 1) / kWave;
     int rc = dispatch_storage(storage, [&](auto S) {
         st = dispatch_variant(variant, [&](auto V) {
             // (dt: see sqrt_time)
             const bool fast = a.e.dt >= 0x1.0p-20f && fast_index_verified(a.e.dt, a.e.tau, stream);
             dispatch_window(a.e.w, fast, [&](auto Wc) {
-                constexpr int VV = decltype(V)::value;
-                hipLaunchKernelGGL((sf_semblance_kernel<MODEL,
-                                                        window_of<decltype(Wc)::value, VV, true>(),
-                                                        VV, decltype(S)::value>),
-                                   dim3((unsigned)blocks), dim3(threads), lds, stream, a);
+                constexpr int VV = decltype(V)::value,
+                              WW = window_of<decltype(Wc)::value, VV, true>();
+                const int waves = std::min(sf_waves<MODEL, WW, VV>((long long)blocks), need);
+                hipLaunchKernelGGL((sf_semblance_kernel<MODEL, WW, VV, decltype(S)::value>),
+                                   dim3((unsigned)blocks), dim3((unsigned)(waves * kWave)), lds,
+                                   stream, a);
             });
         });
     });
