@@ -77,6 +77,7 @@ struct DeArgs {
     float lo[3], hi[3];
     uint32_t key0, key1, stream_base;
     int ntiles;
+    int tl;           // de_spread_kernel: log2 of the t0 samples per workgroup
     float *ws;        // [n*ntiles][2][NP][D+2][64]
     float *result;    // [n][2+D][ns]
     float *pop_x;     // [n][ns][NP][D] or NULL
@@ -360,10 +361,10 @@ __attribute__((amdgpu_waves_per_eu(de_min_occupancy<MODEL, W, VARIANT>(), 8))) v
     de_report<D>(a, g, s, rec);
 }
 
-// The same run spread over more of the chip: a workgroup takes T = 16 consecutive t0 samples,
-// and a wave's lanes split into four groups with an individual each, so that (with up to
-// twelve waves) the whole population of a sample is evaluated at once, one individual per
-// lane.  Workspace rows, random streams, donors and selections are those of
+// The same run spread over more of the chip: a workgroup takes T = 16 consecutive t0 samples
+// (de_spread_shape), and a wave's lanes split into four groups with an individual each, so that
+// (with up to twelve waves) the whole population of a sample is evaluated at once, one
+// individual per lane.  Workspace rows, random streams, donors and selections are those of
 // de_semblance_kernel, so the results are the same bits, and a run may change kernels between
 // generation ranges.
 //
@@ -377,9 +378,7 @@ __attribute__((amdgpu_waves_per_eu(de_min_occupancy<MODEL, W, VARIANT>(), 8))) v
 // midpoints: 62.3 against 67.5 ms here; 32 midpoints, 512 workgroups: 90.5 against 88.4), so
 // it keeps de_semblance_kernel above 512 workgroups of it.  (OCT at T = 8/16/32: 77.8/68.4/
 // 72.6 ms; at eight waves, two passes over 48 individuals, 84.7; at five waves per SIMD 88.8.)
-constexpr int kDeSpreadTl = 4;
 constexpr int kDeSpreadWaves = 12;
-constexpr long long kDeSpreadZocrsTiles = 512;
 template <int MODEL>
 constexpr bool de_spread_always() { return MODEL != HSS_ZOCRS; }
 
@@ -390,7 +389,7 @@ __attribute__((amdgpu_waves_per_eu(6, 8))) void de_spread_kernel(DeArgs a) {
     constexpr int REC = D + 2;  // D parameters, S, stack
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
-    constexpr int T = 1 << kDeSpreadTl;
+    const int T = 1 << a.tl;
     const int wg_per_mid = (a.e.ns + T - 1) / T;
     const int blk = logical_block(blockIdx.x, gridDim.x);
     const int slot = blk / wg_per_mid;
@@ -404,9 +403,9 @@ __attribute__((amdgpu_waves_per_eu(6, 8))) void de_spread_kernel(DeArgs a) {
     const EvalCtx e = midpoint_ctx(a.e, a.mbeg, a.mcnt, a.mm0, g);
     const uint32_t stream = a.stream_base + (uint32_t)g;
     const int NP = a.NP;
-    constexpr int per_wave = kWave / T;
+    const int per_wave = kWave >> a.tl;
     const int per_pass = per_wave * ((int)blockDim.x / kWave);
-    const int first = wave * per_wave + lane / T;  // the lane's individual of a pass
+    const int first = wave * per_wave + (lane >> a.tl);  // the lane's individual of a pass
     // the workspace column of sample s in de_semblance_kernel's 64-sample tiles
     float *const column = a.ws +
                           ((size_t)g * a.ntiles + s0 / kWave) * 2 * NP * REC * kWave + s % kWave;
@@ -464,6 +463,7 @@ __attribute__((amdgpu_waves_per_eu(6, 8))) void de_spread_kernel(DeArgs a) {
     for (int gen = a.gen_begin; gen < a.gen_end; ++gen) {
         const int cur = (gen - 1) & 1, next = gen & 1;
         for (int p0 = 0; p0 < NP; p0 += per_pass) {
+            if (p0 + wave * per_wave >= NP) continue;  // (the whole wave)
             // (a lane past the population works on the last individual and keeps nothing; so
             // does one past the trace, whose column lies in the last tile's padding)
             const bool on = p0 + first < NP;
@@ -515,19 +515,54 @@ __attribute__((amdgpu_waves_per_eu(6, 8))) void de_spread_kernel(DeArgs a) {
     de_report<D>(a, g, s, rec);
 }
 
+// The shape of a de_spread_kernel launch: T = 2^tl samples per workgroup, and its waves.  A CU's
+// four SIMDs share them, so more than four are a multiple of four: as many as take the
+// population in the fewest passes, the last ones idle.  (Five to seven or nine to eleven load the
+// SIMDs unevenly: 100 midpoints, 8 generations, nine | twelve waves for a population of 36, CMP,
+// FP32 3.65 | 3.39 ms; OCT, 30 midpoints, FP16, 4 generations 6.5 | 5.9; ZO-CRS, 20 midpoints,
+// BF16, ten | twelve for 40 8.4 | 6.5.)  CMP launches that fill the chip take workgroups of four,
+// which leave the SIMDs even whatever the population (300 midpoints, 6 generations, 36
+// individuals, nine | twelve | four waves: FP16 10.6 | 9.5 | 7.7 ms, EXACT 16.7 | 14.9 | 12.1; 48
+// individuals, twelve | four: FP16 10.3 | 9.6), FP32 ones once they are large (100 midpoints, 36
+// individuals, twelve | four 3.39 | 3.56, 300 midpoints 7.70 | 7.40); 17 to 24 individuals of a
+// 16-bit line then go eight at a time, not sixteen (FP16, w = 5, 120 midpoints, 20 individuals
+// 2.51 | 2.22 ms).
+struct DeSpreadShape {
+    int tl, waves;
+};
+inline DeSpreadShape de_spread_shape(int model, int storage, int NP, long long n_mid, int ns) {
+    constexpr int tl = 4, per_wave = kWave >> tl;
+    const int need = (NP + per_wave - 1) / per_wave;
+    if (need <= 4) return {tl, need};
+    const long long workgroups = n_mid * ((ns + (1 << tl) - 1) >> tl);
+    if (model == HSS_CMP && workgroups >= (storage == HSS_F32 || need % 4 == 0 ? 8192 : 1536))
+        return {need <= 6 && storage != HSS_F32 ? tl + 1 : tl, 4};
+    const int passes = (need + kDeSpreadWaves - 1) / kDeSpreadWaves;
+    return {tl, ((need + passes - 1) / passes + 3) / 4 * 4};
+}
+
+// Whether ZO-CRS takes de_spread_kernel: up to 512 workgroups of de_semblance_kernel, 400 where
+// some of its waves idle or, three of them, load the SIMDs unevenly (BF16, 36 individuals on nine
+// of twelve waves, it | de_semblance_kernel: 30 midpoints, 480 workgroups 11.7 | 10.3 ms, 24 of
+// them, FP32, 5.2 | 6.7).
+constexpr long long kDeSpreadZocrsTiles = 512, kDeSpreadZocrsTilesIdle = 400;
+inline bool de_spread_zocrs(long long tiles, int NP, DeSpreadShape shape) {
+    const int need = (NP + (kWave >> shape.tl) - 1) / (kWave >> shape.tl);
+    const bool even = need % shape.waves == 0 && shape.waves != 3;
+    return tiles <= (even ? kDeSpreadZocrsTiles : kDeSpreadZocrsTilesIdle);
+}
+
 template <int MODEL>
-int launch_de(const DeArgs &a, int n_mid, int variant, int storage, hipStream_t stream) {
+int launch_de(const DeArgs &args, int n_mid, int variant, int storage, hipStream_t stream) {
     int st = HSS_OK;
+    DeArgs a = args;
     const unsigned blocks = (unsigned)n_mid * (unsigned)a.ntiles;
     if (blocks == 0) return HSS_OK;
-    constexpr int T = 1 << kDeSpreadTl, per_wave = kWave / T;
-    const long long spread = (long long)n_mid * ((a.e.ns + T - 1) / T);
-    const bool spread_it = (de_spread_always<MODEL>() || (long long)blocks <= kDeSpreadZocrsTiles) &&
+    const DeSpreadShape shape = de_spread_shape(MODEL, storage, a.NP, n_mid, a.e.ns);
+    a.tl = shape.tl;
+    const long long spread = (long long)n_mid * ((a.e.ns + (1 << a.tl) - 1) >> a.tl);
+    const bool spread_it = (de_spread_always<MODEL>() || de_spread_zocrs(blocks, a.NP, shape)) &&
                            spread <= 0x7fffffffll;
-    // the waves that take the population in the fewest equal passes
-    const int need = (a.NP + per_wave - 1) / per_wave;
-    const int passes = (need + kDeSpreadWaves - 1) / kDeSpreadWaves;
-    const int waves = (need + passes - 1) / passes;
     int st_launch = HSS_OK;
     int rc = dispatch_storage(storage, [&](auto S) {
         st = dispatch_variant(variant, [&](auto V) {
@@ -537,7 +572,7 @@ int launch_de(const DeArgs &a, int n_mid, int variant, int storage, hipStream_t 
                 if constexpr (WW > 0 && VV != HSS_KAHAN) {
                     if (spread_it) {
                         hipLaunchKernelGGL((de_spread_kernel<MODEL, WW, VV, SS>),
-                                           dim3((unsigned)spread), dim3(waves * kWave), 0, stream,
+                                           dim3((unsigned)spread), dim3(shape.waves * kWave), 0, stream,
                                            a);
                         return;
                     }
