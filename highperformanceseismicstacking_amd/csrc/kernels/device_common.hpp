@@ -180,7 +180,8 @@ template <bool FAST, bool SHIFT>
 __device__ __forceinline__ float sqrt_time(float x) {
     if constexpr (!FAST) return sqrtf(x);
     const float r = sqrt_rn_big(x);
-    if constexpr (SHIFT) return x < 0x1.0p-96f ? 0.0f : r;
+    // (as bit patterns: a negative radicand compares above, and keeps its NaN)
+    if constexpr (SHIFT) return __float_as_uint(x) < 0x0f800000u ? 0.0f : r;
     return r;
 }
 
