@@ -60,18 +60,31 @@ constexpr float kTuneMargin = 0.01f;
 // (code load) covers a sixteenth of that
 constexpr unsigned kTuneBlocks = 8192;
 
-// The compensated variant's shape without timing.  CMP: up to 9 samples the staged kernel with
-// two candidates, at 11 with one, where two spill; at 13 and 15, where both spill, with two
-// from nine rounds on, in FP32 only while workgroups are few.  Else one candidate with direct
-// reads.
-// Direct | staged, 640 samples, 60 traces, 300 candidates, in ms: FP32, 250 midpoints, 5
-// samples 3.11 | 2.56, 9 samples 4.22 | 3.18, 11 samples 3.94 | 4.03, 15 samples 5.00 | 5.79;
-// 16 midpoints, 9 samples 1.12 | 0.47, 11 samples 1.02 | 0.72, 15 samples 1.15 | 0.63; FP16,
-// 250 midpoints, 9 samples 5.58 | 3.14, 11 samples 5.32 | 3.98, 15 samples 6.24 | 5.82.
+// The compensated variant's shape without timing.  CMP, up to 9 samples: the staged kernel with
+// two candidates.  From 11 on its sums spill with two, or read the stage for few: staged with one
+// at 11, and at 13 for few candidates; FP32 takes direct reads once the launch fills the chip.
+// 640 samples, 60 traces, direct | staged with one | with two, in ms:
+//   FP32, w = 11, 60 midpoints, 300 candidates 1.47 | 1.29 | 1.44, 250 midpoints, 90 candidates
+//     1.27 | 1.36 | 1.63, 300 candidates 3.95 | 3.97 | 4.68
+//   FP32, w = 13, 16 midpoints, 40 candidates 0.170 | 0.145 | 0.120, 60 midpoints, 90 candidates
+//     0.537 | 0.533 | 0.568, 250 midpoints, 300 candidates 4.77 | 5.49 | 5.27
+//   FP32, w = 15, 16 midpoints, 40 candidates 0.179 | 0.159 | 0.128, 60 midpoints, 300 candidates
+//     1.75 | 1.91 | 1.78, 250 midpoints 5.07 | 7.06 | 5.76
+//   FP16, w = 11, 250 midpoints, 300 candidates 5.87 | 4.07 | 4.67
+//   FP16, w = 13, 16 midpoints, 40 candidates 0.317 | 0.152 | 0.140, 250 midpoints, 90 candidates
+//     1.88 | 1.73 | 1.86, 300 candidates 6.33 | 5.51 | 5.27
+//   FP16, w = 15, 16 midpoints, 40 candidates 0.327 | 0.169 | 0.153, 250 midpoints, 40 candidates
+//     0.93 | 1.04 | 1.28, 90 candidates 2.03 | 2.24 | 2.06, 300 candidates 6.72 | 7.12 | 5.79
 GridShape kahan_shape(int model, int w, int storage, long long tiles, int P) {
-    if (model != HSS_CMP || w < 5 || w > 15) return GridShape{1, 1, 0};
-    if (w > 11 && (P <= 128 || (storage == HSS_F32 && tiles > 768))) return GridShape{1, 1, 0};
-    return GridShape{w == 11 ? 1 : 2, 1, 1};
+    constexpr GridShape direct{1, 1, 0}, staged_one{1, 1, 1}, staged_two{2, 1, 1};
+    if (model != HSS_CMP || w < 5 || w > 15) return direct;
+    if (w <= 9) return staged_two;
+    if (storage == HSS_F32) {
+        if (w == 11) return tiles > 768 ? direct : staged_one;
+        return tiles > 480 ? direct : staged_two;
+    }
+    if (w == 11 || (w == 13 && P <= 128)) return staged_one;
+    return w == 15 && P <= 64 && tiles > 768 ? direct : staged_two;
 }
 }  // namespace
 
