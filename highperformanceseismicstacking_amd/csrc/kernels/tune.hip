@@ -10,15 +10,17 @@
 //    waves split into TT tiles x 4/TT candidate groups, trading the number of workgroups
 //    per midpoint (and so how a midpoint's work spreads over the CUs of its XCD) against
 //    the candidates each wave walks;
-//  * staging (CMP, one t0 tile per workgroup): the four waves walk the traces together and
+//  * staging (CMP, one t0 tile per workgroup): eight waves walk the traces together and
 //    read their windows from the workgroup's LDS copy of each trace's span, instead of
 //    each lane (FP32) or each wave (16-bit) reading its own.
 // Which shape wins depends on the model, the window size, the storage and the variant.
-// The first launch for a key (device, model, w, variant, storage) that is large enough
-// to time reliably runs every shape on a leading part of the caller's own batch (its
-// first launch slots, about 8192 workgroups), timed with HIP events on the caller's
-// stream, and keeps the fastest (ties within 1% to the preferred shape); later launches
-// reuse it.  The kernels are pure functions
+// Which shape wins also depends on the number of candidates, which the waves take in rounds,
+// and on the launch's size.  The first launch for a key (device, model, w, variant, storage,
+// and up to 64, up to 128 or more candidates) that is large enough to time reliably runs every
+// shape on a leading part of the caller's own batch (its first launch slots, about 8192
+// workgroups), timed with HIP events on the caller's stream, and keeps the fastest (ties within
+// 1% to the preferred shape); later launches that are large enough themselves reuse it, smaller
+// ones take the untuned shape.  The kernels are pure functions
 // of their inputs, so the timing runs write the same outputs (accumulating outputs are
 // withheld from them by the caller).  No tuning under stream capture (the default shape
 // is used), and HSS_AUTOTUNE=0 in the environment turns tuning off.
@@ -29,6 +31,7 @@
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <utility>
 
 #include "launch_util.hpp"
 
@@ -36,11 +39,12 @@ namespace hss {
 
 namespace {
 std::mutex tune_mu;
-struct TunedShape {
-    GridShape shape;
-    bool pinned;  // by hss_grid_set_shape
-};
-std::map<std::tuple<int, int, int, int, int>, TunedShape> tune_cache;
+using TuneKey = std::tuple<int, int, int, int, int>;      // device, model, w, variant, storage
+std::map<TuneKey, GridShape> pinned_shapes;               // by hss_grid_set_shape
+std::map<std::pair<TuneKey, int>, GridShape> timed_shapes;  // by candidate_class() too
+
+constexpr int kCandidateClasses = 3;
+int candidate_class(int P) { return P <= 64 ? 0 : (P <= 128 ? 1 : 2); }
 
 bool tuning_enabled() {
     const char *v = std::getenv("HSS_AUTOTUNE");
@@ -59,6 +63,8 @@ constexpr float kTuneMargin = 0.01f;
 // workgroups a timing run covers (a leading part of the batch); the warm-up run before it
 // (code load) covers a sixteenth of that
 constexpr unsigned kTuneBlocks = 8192;
+// workgroups of a launch that times reliably (several waves of them per CU)
+constexpr unsigned kTuneLeast = 4096;
 
 // The compensated variant's shape without timing.  CMP, up to 9 samples: the staged kernel with
 // two candidates.  From 11 on its sums spill with two, or read the stage for few: staged with one
@@ -93,12 +99,19 @@ int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, in
                      GridShape *shape_out) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) dev = -1;
-    const auto key = std::make_tuple(dev, model, w, variant, storage);
+    const TuneKey key(dev, model, w, variant, storage);
+    const auto timed_key = std::make_pair(key, candidate_class(P));
+    const unsigned long long blocks = (unsigned long long)n_slots * (unsigned long long)ntiles;
     {
         std::lock_guard<std::mutex> lock(tune_mu);
-        auto it = tune_cache.find(key);
-        if (it != tune_cache.end()) {
-            *shape_out = it->second.shape;
+        auto pin = pinned_shapes.find(key);
+        if (pin != pinned_shapes.end()) {
+            *shape_out = pin->second;
+            return HSS_OK;
+        }
+        auto it = timed_shapes.find(timed_key);
+        if (blocks >= kTuneLeast && it != timed_shapes.end()) {
+            *shape_out = it->second;
             return HSS_OK;
         }
     }
@@ -110,9 +123,7 @@ int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, in
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
         return HSS_OK;
-    // only launches with several waves of workgroups per CU time reliably
-    const unsigned long long blocks = (unsigned long long)n_slots * (unsigned long long)ntiles;
-    if (!tuning_enabled() || blocks < 4096) return HSS_OK;
+    if (!tuning_enabled() || blocks < kTuneLeast) return HSS_OK;
     const int slots = (int)std::min<unsigned long long>(
         (unsigned long long)n_slots, (kTuneBlocks + ntiles - 1) / (unsigned)ntiles);
     hipEvent_t e0, e1;
@@ -146,32 +157,37 @@ int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, in
     if (rc != HSS_OK) return rc;
     if (!timed) return HSS_OK;  // a HIP call failed: keep the default, cache nothing
     std::lock_guard<std::mutex> lock(tune_mu);
-    tune_cache[key] = TunedShape{best, false};
+    timed_shapes[timed_key] = best;
     *shape_out = best;
     return HSS_OK;
 }
 
 void tuned_grid_store(int dev, int model, int w, int variant, int storage, GridShape shape) {
     std::lock_guard<std::mutex> lock(tune_mu);
-    const auto key = std::make_tuple(dev, model, w, variant, storage);
-    if (shape.cpl == 0)
-        tune_cache.erase(key);
-    else
-        tune_cache[key] = TunedShape{shape, true};
+    const TuneKey key(dev, model, w, variant, storage);
+    pinned_shapes.erase(key);
+    for (int c = 0; c < kCandidateClasses; ++c) timed_shapes.erase({key, c});
+    if (shape.cpl != 0) pinned_shapes[key] = shape;
 }
 
+// The pinned shape, else the one timed for the most candidates.
 GridShape tuned_grid_lookup(int dev, int model, int w, int variant, int storage) {
     std::lock_guard<std::mutex> lock(tune_mu);
-    auto it = tune_cache.find(std::make_tuple(dev, model, w, variant, storage));
-    return it == tune_cache.end() ? GridShape{0, 0, 0} : it->second.shape;
+    const TuneKey key(dev, model, w, variant, storage);
+    auto pin = pinned_shapes.find(key);
+    if (pin != pinned_shapes.end()) return pin->second;
+    for (int c = kCandidateClasses - 1; c >= 0; --c) {
+        auto it = timed_shapes.find({key, c});
+        if (it != timed_shapes.end()) return it->second;
+    }
+    return GridShape{0, 0, 0};
 }
 
 bool grid_shape_pinned(int model, int w, int variant, int storage) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return false;
     std::lock_guard<std::mutex> lock(tune_mu);
-    auto it = tune_cache.find(std::make_tuple(dev, model, w, variant, storage));
-    return it != tune_cache.end() && it->second.pinned;
+    return pinned_shapes.count(TuneKey(dev, model, w, variant, storage)) != 0;
 }
 
 }  // namespace hss
