@@ -365,7 +365,7 @@ __attribute__((amdgpu_waves_per_eu(staged_min_waves<W, VARIANT, CPL>(), 8))) voi
         }
     }
 
-    // the four waves' bests of each t0, as merge_bests merges them (the largest value, the
+    // the waves' bests of each t0, as merge_bests merges them (the largest value, the
     // smallest candidate index among equal values)
     __syncthreads();
     if (wave != 0 || !active) return;

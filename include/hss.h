@@ -179,25 +179,29 @@ int hss_grid_semblance_plain(const hss_traces *traces, int model, const float *d
                              const int32_t *h_count, const float *h_m0, float h0, float apm,
                              float *d_sembl, float *d_stack, float *d_result, void *stream);
 
-/* Launch shapes of the grid search.  Unless a shape is pinned for the key (below), ZO-CRS and
- * OCT launches and small CMP launches (up to 768 64-sample tiles over all midpoints, 240 with
- * 16-bit storage) of a compiled window size and without compensation take a kernel whose
- * shape follows from the launch's size, and tune nothing.
+/* Launch shapes of the grid search.  Unless a shape is pinned for the key (below), launches of a
+ * compiled window size (odd, 3 to 31) and without compensation take a kernel whose shape follows
+ * from the launch's size, and tune nothing: ZO-CRS and OCT always, CMP up to 320 64-sample tiles
+ * over all midpoints (160 with 16-bit storage).  For the others:
  *
  * The launch shape the grid-search autotuner chose on the current device for (model, w,
  * variant, storage): *cpl = candidates per lane (1 or 2), *t0_tiles = 64-sample t0 tiles
- * per workgroup (1, 2 or 4; the workgroup's four waves split into that many tiles times
- * 4 / t0_tiles candidate groups), *staged = 1 when the workgroup stages each trace's span
- * in LDS for all its waves (CMP, one t0 tile per workgroup); all 0 when that key has not
- * been tuned yet.  No
+ * per workgroup (1, 2 or 4; an unstaged workgroup's four waves split into that many tiles
+ * times 4 / t0_tiles candidate groups), *staged = 1 when a workgroup, of eight waves then,
+ * stages each trace's span in LDS for all of them (CMP, one t0 tile per workgroup); all 0 when
+ * that key has not been tuned.  Shapes are timed for up to 64, up to 128 and more candidates
+ * apart; the one for the most is reported.  No
  * counterpart in the reference.  hss_grid_semblance tunes on its first launch of at
  * least 4096 workgroups for a key (outside stream capture) by timing each shape (six
  * unstaged, and for CMP two staged) on the first launch slots of the caller's batch
  * (about 8192 workgroups) and keeping the fastest, a shape listed earlier (two candidates
- * per lane, one t0 tile, unstaged first) winning ties within 1%; the environment variable
- * HSS_AUTOTUNE=0 turns it off.  An untuned launch runs two candidates per lane, one t0
- * tile, staged for CMP (HSS_KAHAN: one candidate, unstaged).  Results do not depend on the
- * shape (bit for bit). */
+ * per lane, one t0 tile, unstaged first) winning ties within 1%; launches of at least that
+ * size reuse it, but that few candidates (up to 72) of a staged launch go one to a lane
+ * whatever was timed.  The environment variable
+ * HSS_AUTOTUNE=0 turns it off.  Any other launch runs two candidates per lane, one t0
+ * tile, staged for CMP; HSS_KAHAN: one candidate, unstaged, but for CMP windows of 5 to 15
+ * samples, which are staged with one or two where that is faster (up to 9 samples always).
+ * Results do not depend on the shape (bit for bit). */
 int hss_grid_tuned_shape(int model, int w, int variant, int storage, int32_t *cpl,
                          int32_t *t0_tiles, int32_t *staged);
 /* hss_grid_tuned_shape's candidates per lane only. */
