@@ -117,9 +117,15 @@ int tuned_grid_shape(int model, int w, int variant, int storage, int n_slots, in
     }
     // untuned launches (small, under capture, tuning off): the choice of every tuned line
     // -- two candidates per lane, for CMP with the workgroup-staged traces -- but for the
-    // compensated variant
-    *shape_out = variant == HSS_KAHAN ? kahan_shape(model, w, storage, (long long)n_slots * ntiles, P)
-                                      : GridShape{2, 1, model == HSS_CMP ? 1 : 0};
+    // compensated variant, and for up to 24 candidates of FP32 windows of 5 and 7 samples in
+    // large launches, where a round or two of the staged kernel's eight waves do not pay for the
+    // stage (400 midpoints of 640 samples, 24 candidates, staged | direct, w = 5 0.323 | 0.301,
+    // w = 7 0.363 | 0.322 ms; 32 candidates, w = 5 0.382 | 0.397; 60 midpoints, EXACT, w = 5, 24
+    // candidates 0.085 | 0.097)
+    const bool few = model == HSS_CMP && storage == HSS_F32 && (w == 5 || w == 7) && P <= 24 &&
+                     blocks > 1200;
+    *shape_out = variant == HSS_KAHAN ? kahan_shape(model, w, storage, (long long)blocks, P)
+                                      : GridShape{2, 1, model == HSS_CMP && !few ? 1 : 0};
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
         return HSS_OK;
